@@ -34,22 +34,18 @@ __host__ __device__ constexpr bool qtype_supported(int qt) { return group_bytes(
 typedef uint16_t bf16_t;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// Exact fp16 -> fp32 (normals by re-biasing, subnormals as man * 2^-24).
-__device__ __forceinline__ float h2f(uint32_t h) {
-    const uint32_t sign = (h & 0x8000u) << 16;
-    const uint32_t em = h & 0x7fffu;
-    if (em >= 0x0400u) {
-        const uint32_t bits = em >= 0x7c00u ? (0x7f800000u | ((em & 0x3ffu) << 13)) : ((em << 13) + 0x38000000u);
-        return __uint_as_float(bits | sign);
-    }
-    return __uint_as_float(sign | __float_as_uint((float)em * 5.9604644775390625e-8f));
-}
-
 // Hardware fp16 -> fp32 (v_cvt_f32_f16): exact for normals, subnormals and
 // infinities; a NaN stays a NaN but its payload may be quieted, so only paths
-// whose output does not carry NaN payloads (the bf16 mixture) use it.
+// whose output does not carry NaN payloads (the bf16 mixture, dots) use it.
 __device__ __forceinline__ float h2f_hw(uint32_t h) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
+}
+
+// Exact fp16 -> fp32, NaN payloads included; no branch, so the loads of
+// neighbouring runs are not held back by one.
+__device__ __forceinline__ float h2f(uint32_t h) {
+    const uint32_t nan = 0x7f800000u | ((h & 0x3ffu) << 13) | ((h & 0x8000u) << 16);
+    return (h & 0x7fffu) > 0x7c00u ? __uint_as_float(nan) : h2f_hw(h);
 }
 
 // fp32 -> bf16 exactly as torch's Float->BFloat16 cast: NaN -> 0x7FC0, else
@@ -106,21 +102,32 @@ struct HasMin {
     static constexpr bool value = (QT == Q4_K || QT == Q5_K || QT == Q2_K);
 };
 
-// 6-bit scale/min pair j of the 12-byte Q4_K/Q5_K scale array
+// 6-bit scale/min pair j of the 12-byte Q4_K/Q5_K scale array (4-byte aligned),
+// from its three words: no branch on j, and one wide read for the whole array.
 __device__ __forceinline__ void scale_min_k4(const uint8_t* __restrict__ s, int j, uint32_t& sc, uint32_t& m) {
-    if (j < 4) {
-        sc = s[j] & 63u;
-        m = s[j + 4] & 63u;
-    } else {
-        sc = (s[j + 4] & 0xFu) | ((uint32_t)(s[j - 4] >> 6) << 4);
-        m = (s[j + 4] >> 4) | ((uint32_t)(s[j] >> 6) << 4);
-    }
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(s);
+    const int sh = 8 * (j & 3);
+    const uint32_t b0 = w[0] >> sh, b1 = w[1] >> sh, b2 = w[2] >> sh;  // byte j % 4 of each word, in the low bits
+    const bool low = j < 4;
+    sc = low ? b0 & 63u : (b2 & 0xFu) | ((b0 >> 2) & 0x30u);
+    m = low ? b1 & 63u : ((b2 >> 4) & 0xFu) | ((b1 >> 2) & 0x30u);
+}
+
+// 6-bit scale is (0..15) of the 12-byte Q3_K scale array, biased by 32.
+__device__ __forceinline__ uint32_t scale_q3k(const uint8_t* __restrict__ s, int is) {
+    const uint32_t lo4 = ((uint32_t)s[is & 7] >> (4 * (is >> 3))) & 0xFu;
+    const uint32_t hi2 = ((uint32_t)s[8 + (is & 3)] >> (2 * (is >> 2))) & 3u;
+    return lo4 | (hi2 << 4);
 }
 
 // Load R (4, 8 or 16) consecutive bytes whose address is a multiple of ALIGN
 // (a property of the format's layout: group bases are 16-byte aligned in
 // memory and in LDS, so field offsets fix the alignment), with the widest
 // loads that alignment allows.  Byte r is (w[r / 4] >> (8 * (r % 4))) & 0xff.
+// At 2-byte alignment the run is cut out of the aligned words that hold it
+// (never one past the run's last byte): R / 4 + 1 word reads and R / 4 byte
+// shifts, where halves took R / 2 reads and R / 4 merges and the LDS
+// instructions, not the bytes, set the pace.
 template <int ALIGN, int R>
 __device__ __forceinline__ void load_run(const uint8_t* __restrict__ p, uint32_t (&w)[R / 4]) {
     if constexpr (ALIGN >= 8 && R % 8 == 0) {
@@ -134,9 +141,14 @@ __device__ __forceinline__ void load_run(const uint8_t* __restrict__ p, uint32_t
 #pragma unroll
         for (int i = 0; i < R / 4; ++i) w[i] = *reinterpret_cast<const uint32_t*>(p + 4 * i);
     } else {
-        const uint16_t* h = reinterpret_cast<const uint16_t*>(p);
+        const int over = (int)(reinterpret_cast<uintptr_t>(p) & 3u);  // 0 or 2
+        const uint8_t* base = p - over;
+        uint32_t x[R / 4 + 1];
 #pragma unroll
-        for (int i = 0; i < R / 4; ++i) w[i] = (uint32_t)h[2 * i] | ((uint32_t)h[2 * i + 1] << 16);
+        for (int i = 0; i < R / 4; ++i) x[i] = *reinterpret_cast<const uint32_t*>(base + 4 * i);
+        x[R / 4] = *reinterpret_cast<const uint32_t*>(base + R - 4 + 2 * over);
+#pragma unroll
+        for (int i = 0; i < R / 4; ++i) w[i] = __builtin_amdgcn_alignbyte(x[i + 1], x[i], over);
     }
 }
 
@@ -155,9 +167,11 @@ __device__ __forceinline__ uint32_t run_byte(const uint32_t (&w)[R / 4], int r) 
     return (w[r >> 2] >> (8 * (r & 3))) & 0xffu;
 }
 
-template <int QT, int R>
+template <int QT, int R, bool HW = false>
 __device__ __forceinline__ void decode_codes(const uint8_t* __restrict__ g, int p, float* __restrict__ q, float& dl,
                                              float& ml) {
+    // HW: the caller's result carries no NaN payload
+    auto h2f = [](uint32_t h) { return HW ? h2f_hw(h) : vq::h2f(h); };
     if constexpr (QT == Q8_0) {
         // blocks of 34 bytes: codes start 2 bytes into a block -> 2-byte aligned
         const uint8_t* b = g + 34 * (p >> 5);
@@ -205,10 +219,7 @@ __device__ __forceinline__ void decode_codes(const uint8_t* __restrict__ g, int 
         const float d = h2f(*reinterpret_cast<const uint16_t*>(g + 108));
         const int n = p >> 7, j = (p >> 5) & 3, half = (p >> 4) & 1, l = p & 15;
         const int is = 8 * n + 2 * j + half;
-        const uint8_t* s = g + 96;
-        const uint32_t lo4 = is < 8 ? (s[is] & 0xFu) : (uint32_t)(s[is - 8] >> 4);
-        const uint32_t hi2 = (s[8 + (is & 3)] >> (2 * (is >> 2))) & 3u;
-        dl = d * (float)((int)(lo4 | (hi2 << 4)) - 32);
+                dl = d * (float)((int)scale_q3k(g + 96, is) - 32);
         ml = 0.0f;
         uint32_t qw[R / 4], mw[R / 4];
         load_run<2, R>(g + 32 + 32 * n + 16 * half + l, qw);
@@ -252,7 +263,7 @@ __device__ __forceinline__ void decode_run(const uint8_t* __restrict__ g, int p,
 template <int QT, int R>
 __device__ __forceinline__ float dot_run(const uint8_t* __restrict__ g, int p, const float* __restrict__ v) {
     float q[R], dl, ml;
-    decode_codes<QT, R>(g, p, q, dl, ml);
+    decode_codes<QT, R, true>(g, p, q, dl, ml);
     float s1 = 0.0f, s0 = 0.0f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -284,18 +295,18 @@ __device__ __forceinline__ float dot_sub16(const uint8_t* __restrict__ g, int p,
     const int l = p & 16;  // first weight within the 32-weight run
     if constexpr (QT == Q8_0) {
         const uint8_t* b = g + 34 * (p >> 5);
-        dl = h2f(*reinterpret_cast<const uint16_t*>(b));
-        const uint16_t* q = reinterpret_cast<const uint16_t*>(b + 2 + l);  // 2-byte aligned
+        dl = h2f_hw(*reinterpret_cast<const uint16_t*>(b));
+        load_run<2, 16>(b + 2 + l, uw);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) uw[u] = ((uint32_t)q[2 * u] | ((uint32_t)q[2 * u + 1] << 16)) ^ 0x80808080u;
+        for (int u = 0; u < 4; ++u) uw[u] ^= 0x80808080u;
         off = 128.0f;
     } else if constexpr (QT == Q4_K || QT == Q5_K) {
         const uint32_t dd = *reinterpret_cast<const uint32_t*>(g);
         const int c = p >> 6, nib = (p >> 5) & 1;
         uint32_t sc, m;
         scale_min_k4(g + 4, 2 * c + nib, sc, m);
-        dl = h2f(dd & 0xffffu) * (float)sc;
-        ml = h2f(dd >> 16) * (float)m;
+        dl = h2f_hw(dd & 0xffffu) * (float)sc;
+        ml = h2f_hw(dd >> 16) * (float)m;
         // 144- and 176-byte groups keep 16-byte alignment
         const u32x4 w = *reinterpret_cast<const u32x4*>(g + (QT == Q5_K ? 48 : 16) + 32 * c + l);
 #pragma unroll
@@ -307,43 +318,35 @@ __device__ __forceinline__ float dot_sub16(const uint8_t* __restrict__ g, int p,
             for (int u = 0; u < 4; ++u) uw[u] |= ((x[u] >> xs) & 0x01010101u) << 4;
         }
     } else if constexpr (QT == Q6_K) {
-        const float d = h2f(*reinterpret_cast<const uint16_t*>(g + 208));
+        const float d = h2f_hw(*reinterpret_cast<const uint16_t*>(g + 208));
         const int n = p >> 7, t4 = (p >> 5) & 3;
         dl = d * (float)(int8_t)g[192 + 8 * n + 2 * t4 + (l >> 4)];
-        const uint16_t* a = reinterpret_cast<const uint16_t*>(g + 64 * n + 32 * (t4 & 1) + l);  // 2-byte aligned
-        const uint16_t* b = reinterpret_cast<const uint16_t*>(g + 128 + 32 * n + l);
+        uint32_t lw[4], hw[4];
+        load_run<2, 16>(g + 64 * n + 32 * (t4 & 1) + l, lw);
+        load_run<2, 16>(g + 128 + 32 * n + l, hw);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint32_t lw = (uint32_t)a[2 * u] | ((uint32_t)a[2 * u + 1] << 16);
-            const uint32_t hw = (uint32_t)b[2 * u] | ((uint32_t)b[2 * u + 1] << 16);
-            uw[u] = ((lw >> (4 * (t4 >> 1))) & 0x0F0F0F0Fu) | (((hw >> (2 * t4)) & 0x03030303u) << 4);
-        }
+        for (int u = 0; u < 4; ++u)
+            uw[u] = ((lw[u] >> (4 * (t4 >> 1))) & 0x0F0F0F0Fu) | (((hw[u] >> (2 * t4)) & 0x03030303u) << 4);
         off = 32.0f;
     } else if constexpr (QT == Q3_K) {
-        const float d = h2f(*reinterpret_cast<const uint16_t*>(g + 108));
+        const float d = h2f_hw(*reinterpret_cast<const uint16_t*>(g + 108));
         const int n = p >> 7, j = (p >> 5) & 3;
-        const uint8_t* sb = g + 96;
         const int is = 8 * n + 2 * j + (l >> 4);
-        const uint32_t lo4 = is < 8 ? (sb[is] & 0xFu) : (uint32_t)(sb[is - 8] >> 4);
-        const uint32_t hi2 = (sb[8 + (is & 3)] >> (2 * (is >> 2))) & 3u;
-        dl = d * (float)((int)(lo4 | (hi2 << 4)) - 32);
-        const uint16_t* a = reinterpret_cast<const uint16_t*>(g + 32 + 32 * n + l);  // 2-byte aligned
-        const uint16_t* b = reinterpret_cast<const uint16_t*>(g + l);
+                dl = d * (float)((int)scale_q3k(g + 96, is) - 32);
+        uint32_t lw[4], hw[4];
+        load_run<2, 16>(g + 32 + 32 * n + l, lw);
+        load_run<2, 16>(g + l, hw);
         const int xs = 4 * n + j;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint32_t lw = (uint32_t)a[2 * u] | ((uint32_t)a[2 * u + 1] << 16);
-            const uint32_t hw = (uint32_t)b[2 * u] | ((uint32_t)b[2 * u + 1] << 16);
-            // q = low2 - (hmask bit ? 0 : 4) = (low2 | bit << 2) - 4
-            uw[u] = ((lw >> (2 * j)) & 0x03030303u) | (((hw >> xs) & 0x01010101u) << 2);
-        }
+        for (int u = 0; u < 4; ++u)  // q = low2 - (hmask bit ? 0 : 4) = (low2 | bit << 2) - 4
+            uw[u] = ((lw[u] >> (2 * j)) & 0x03030303u) | (((hw[u] >> xs) & 0x01010101u) << 2);
         off = 4.0f;
     } else {  // Q2_K: 84-byte groups keep 4-byte alignment
         const uint32_t dd = *reinterpret_cast<const uint32_t*>(g + 80);
         const int n = p >> 7, j = (p >> 5) & 3;
         const uint32_t sc = g[8 * n + 2 * j + (l >> 4)];
-        dl = h2f(dd & 0xffffu) * (float)(sc & 0xFu);
-        ml = h2f(dd >> 16) * (float)(sc >> 4);
+        dl = h2f_hw(dd & 0xffffu) * (float)(sc & 0xFu);
+        ml = h2f_hw(dd >> 16) * (float)(sc >> 4);
         const uint32_t* q = reinterpret_cast<const uint32_t*>(g + 16 + 32 * n + l);
 #pragma unroll
         for (int u = 0; u < 4; ++u) uw[u] = (q[u] >> (2 * j)) & 0x03030303u;
@@ -417,10 +420,7 @@ __device__ __forceinline__ void decode_affine(const uint8_t* __restrict__ g, int
         const float d = h2f_hw(*reinterpret_cast<const uint16_t*>(g + 108));
         const int n = p >> 7, j = (p >> 5) & 3, half = (p >> 4) & 1, l = p & 15;
         const int is = 8 * n + 2 * j + half;
-        const uint8_t* sb = g + 96;
-        const uint32_t lo4 = is < 8 ? (sb[is] & 0xFu) : (uint32_t)(sb[is - 8] >> 4);
-        const uint32_t hi2 = (sb[8 + (is & 3)] >> (2 * (is >> 2))) & 3u;
-        dl = d * (float)((int)(lo4 | (hi2 << 4)) - 32);
+                dl = d * (float)((int)scale_q3k(g + 96, is) - 32);
         c = -4.0f * dl;
         uint32_t hw[W];
         load_run<2, R>(g + 32 + 32 * n + 16 * half + l, uw);

@@ -1,28 +1,8 @@
 // Tile configurations and launchers of the gated-Linear GEMMs (the kernel
 // templates live in vq_gemm_impl.h).
-#include "vq_gemm_impl.h"
+#include "vq_gemm_stream.h"
 
 namespace vq {
-
-// 256x256 output tiles, 8 waves in a 4 x 2 layout (64x128 each, 128 fp32
-// accumulators per lane) and two waves per SIMD, so one wave's fragment reads
-// and copies hide under the other's MFMAs; operands copied global -> LDS by
-// direct-to-LDS loads into two padded LDS stages with the stage switch inside
-// the MFMA stream, BK = 64; the stage-switch order is chosen per product.
-// Measured on MI355X at 8192 tokens against the same tiles with 4 waves of
-// 128x128 and one wave per SIMD: forward 5120 -> 17408 1238 vs 1336 us,
-// 17408 -> 5120 1226 vs 1392 us, 4096 -> 28672 1594 vs 1702 us; dX + gate
-// 2659 vs 2690 us.
-// Operands stored [K][rows] (dX's W, both gate operands) keep that orientation
-// in LDS and are read with ds_read_b64_tr_b16.
-constexpr int kWaves = 8;
-using FwdLA = DmaKS<256, 64, 64 * kWaves>;
-using FwdLB = DmaKS<256, 64, 64 * kWaves>;
-using DxLA = DmaKS<256, 64, 64 * kWaves>;
-using DxLB = DmaNS<256, 64, 64 * kWaves>;
-using GateL = DmaNS<256, 64, 64 * kWaves>;
-using GateLA = DmaNS<256, 64, 64 * kWaves, 1>;  // weight rows permuted for the gate epilogue
-constexpr int kGateBI = 256, kGateBJ = 256;
 
 hipError_t stream_fence(hipStream_t from, hipStream_t to) {
     if (from == to) return hipSuccess;
@@ -63,15 +43,13 @@ int device_cus() {
     return cus;
 }
 
-// Every 8-wave product issues each refill in two halves (COPY_SPLIT) and
-// pins its schedule only at each stage's first k-step (SWITCH_LOOSE).  The
-// forward: split refills 0.3-4% faster at every swept shape, then SWITCH_LOOSE
-// 0.1-1.0% faster than SWITCH_READ_FIRST at 8192 tokens and 5120 -> 17408,
-// 4096 -> 28672, 14336 -> 4096, 1024 -> 6144, 1024 -> 1536.  The backward:
-// 3.0-3.1% faster than dX SWITCH_FREE + gate SWITCH_LOOSE with single-burst
-// refills at 5120 -> 17408, 17408 -> 5120, 4096 -> 28672 (0.6-1.3% at
-// 1024-wide).
-using FwdCfg = GemmCfg<FwdLA, FwdLB, 256, 256, 64, 4, 2, EPI_STORE, 2, SWITCH_LOOSE, 2, COPY_SPLIT>;
+// Y[m][n]: A = W (K-major rows n), B = X; dX[m][d]: A = W ([K = n][d]), B = dY;
+// dW tiles [d][n]: A = X ([K = m][d]), B = dY ([K = m][n]).
+using FwdCfg = StCfg<KS, KS, EPI_STORE>;
+using DxCfg = StCfg<NS, KS, EPI_STORE>;
+using GateCfg = StCfg<NS, NS, EPI_GATE>;
+using GatePartsCfg = StCfg<NS, NS, EPI_PARTS>;
+constexpr int kGateBI = kStTile, kGateBJ = kStTile;
 // Products with fewer 256x256 tiles than three quarters of the CUs (the 0.8B
 // decoder's 1024-wide projections at 8192 tokens) fill the chip better with
 // 128x128 tiles, four waves of 64x64 and two workgroups per CU (measured on
@@ -81,25 +59,27 @@ using FwdCfg = GemmCfg<FwdLA, FwdLB, 256, 256, 64, 4, 2, EPI_STORE, 2, SWITCH_LO
 // than a fenced stage switch with one burst per refill (8192 tokens at
 // 1024 -> 1024, 2048 -> 1024, 3072 -> 1024; 4096 tokens at 1024 -> 1024).
 using FwdSmallCfg =
-    GemmCfg<DmaKS<128, 64, 256>, DmaKS<128, 64, 256>, 128, 128, 64, 2, 2, EPI_STORE, 2, SWITCH_READ_FIRST, 2, COPY_SPLIT>;
+    GemmCfg<DmaKS<128, 64, 256>, DmaKS<128, 64, 256>, 128, 128, 64, 2, 2, 2>;
 
 static bool small_product(int M, int N) {
     const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
     return 4 * tiles < 3 * (int64_t)device_cus();
 }
-using DxCfg = GemmCfg<DxLA, DxLB, 256, 256, 64, 4, 2, EPI_STORE, 2, SWITCH_LOOSE, 2, COPY_SPLIT>;
-using GateCfg = GemmCfg<GateLA, GateL, kGateBI, kGateBJ, 64, 4, 2, EPI_GATE, 2, SWITCH_LOOSE, 2, COPY_SPLIT>;
-using GatePartsCfg = GemmCfg<GateLA, GateL, kGateBI, kGateBJ, 64, 4, 2, EPI_PARTS, 2, SWITCH_LOOSE, 2, COPY_SPLIT>;
-
-static GemmParams fwd_params(const bf16_t* X, const bf16_t* W, int64_t ldw, bf16_t* Y, int M, int N, int D) {
+static GemmParams small_params(const bf16_t* X, const bf16_t* W, int64_t ldw, bf16_t* Y, int M, int N, int D) {
     GemmParams p{};
     p.A = X; p.lda = D; p.B = W; p.ldb = ldw; p.I = M; p.J = N; p.K = D; p.C = Y; p.ldc = N;
     return p;
 }
 
+static GemmParams fwd_params(const bf16_t* X, const bf16_t* W, int64_t ldw, bf16_t* Y, int M, int N, int D) {
+    GemmParams p{};
+    p.A = W; p.lda = ldw; p.B = X; p.ldb = D; p.I = N; p.J = M; p.K = D; p.C = Y; p.ldc = N;
+    return p;
+}
+
 static GemmParams dx_params(const bf16_t* dY, const bf16_t* W, int64_t ldw, bf16_t* dX, int M, int N, int D) {
     GemmParams p{};
-    p.A = dY; p.lda = N; p.B = W; p.ldb = ldw; p.I = M; p.J = D; p.K = N; p.C = dX; p.ldc = D;
+    p.A = W; p.lda = ldw; p.B = dY; p.ldb = N; p.I = D; p.J = M; p.K = N; p.C = dX; p.ldc = D;
     return p;
 }
 
@@ -167,11 +147,12 @@ int64_t dx_tail_bytes(int M, int N, int D) {
 
 // fp32 workspace for the K parts of the forward's split tail tiles.
 int64_t fwd_tail_bytes(int M, int N, int D) {
-    GemmParams p = fwd_params(nullptr, nullptr, 0, nullptr, M, N, D);
     if (small_product(M, N)) {
+        GemmParams p = small_params(nullptr, nullptr, 0, nullptr, M, N, D);
         FwdSmallCfg::plan(p, device_cus(), true);
         return FwdSmallCfg::tail_bytes(p);
     }
+    GemmParams p = fwd_params(nullptr, nullptr, 0, nullptr, M, N, D);
     FwdCfg::plan(p, device_cus(), true);
     return FwdCfg::tail_bytes(p);
 }
@@ -179,13 +160,13 @@ int64_t fwd_tail_bytes(int M, int N, int D) {
 hipError_t launch_gemm_fwd(const bf16_t* X, const bf16_t* W, int64_t ldw, bf16_t* Y, int M, int N, int D,
                            float* tail_ws, hipStream_t s) {
     if (small_product(M, N))
-        return launch_gemm_cfg<FwdSmallCfg>(fwd_params(X, W, ldw, Y, M, N, D), device_cus(), tail_ws, s);
-    return launch_gemm_cfg<FwdCfg>(fwd_params(X, W, ldw, Y, M, N, D), device_cus(), tail_ws, s);
+        return launch_gemm_cfg<FwdSmallCfg>(small_params(X, W, ldw, Y, M, N, D), device_cus(), tail_ws, s);
+    return launch_st_store<FwdCfg>(fwd_params(X, W, ldw, Y, M, N, D), device_cus(), tail_ws, s);
 }
 
 hipError_t launch_gemm_dx(const bf16_t* dY, const bf16_t* W, int64_t ldw, bf16_t* dX, int M, int N, int D,
                           float* tail_ws, hipStream_t s) {
-    return launch_gemm_cfg<DxCfg>(dx_params(dY, W, ldw, dX, M, N, D), device_cus(), tail_ws, s);
+    return launch_st_store<DxCfg>(dx_params(dY, W, ldw, dX, M, N, D), device_cus(), tail_ws, s);
 }
 
 static GemmParams parts_params(const bf16_t* dY, const bf16_t* X, float* dwp, int parts, int M, int N, int D) {
@@ -200,14 +181,14 @@ hipError_t launch_gemm_gate(const bf16_t* dY, const bf16_t* X, const CandGroup& 
     if (dwp) {
         const int np = gate_parts(M, N, D);
         if (np == 0) return hipErrorInvalidValue;
-        hipError_t e = launch_gemm_cfg<GatePartsCfg>(parts_params(dY, X, dwp, np, M, N, D), device_cus(), nullptr, s);
+        hipError_t e = launch_st_gate<GatePartsCfg, false>(parts_params(dY, X, dwp, np, M, N, D), device_cus(), s);
         if (e == hipSuccess) e = stream_fence(s, ds);
         if (e != hipSuccess) return e;
         return launch_gate_dot(cg, N, D, dwp, np, partials, ds);
     }
     if (any_iq(cg))
-        return launch_gemm_cfg<GateCfg, true>(gate_params(dY, X, cg, partials, M, N, D), device_cus(), nullptr, s);
-    return launch_gemm_cfg<GateCfg>(gate_params(dY, X, cg, partials, M, N, D), device_cus(), nullptr, s);
+        return launch_st_gate<GateCfg, true>(gate_params(dY, X, cg, partials, M, N, D), device_cus(), s);
+    return launch_st_gate<GateCfg, false>(gate_params(dY, X, cg, partials, M, N, D), device_cus(), s);
 }
 
 // dX and gate products of one backward in a single launch (dX work items,
@@ -218,7 +199,7 @@ hipError_t launch_gemm_dx_gate(const bf16_t* dY, const bf16_t* W, int64_t ldw, b
     if (dwp) {
         const int np = gate_parts(M, N, D);
         if (np == 0) return hipErrorInvalidValue;
-        hipError_t e = launch_gemm_dual<DxCfg, GatePartsCfg>(dx_params(dY, W, ldw, dX, M, N, D),
+        hipError_t e = launch_st_dual<DxCfg, GatePartsCfg, false>(dx_params(dY, W, ldw, dX, M, N, D),
                                                              parts_params(dY, X, dwp, np, M, N, D), device_cus(),
                                                              tail_ws, s);
         if (e == hipSuccess) e = stream_fence(s, ds);
@@ -226,20 +207,16 @@ hipError_t launch_gemm_dx_gate(const bf16_t* dY, const bf16_t* W, int64_t ldw, b
         return launch_gate_dot(cg, N, D, dwp, np, partials, ds);
     }
     if (any_iq(cg))
-        return launch_gemm_dual<DxCfg, GateCfg, true>(dx_params(dY, W, ldw, dX, M, N, D),
+        return launch_st_dual<DxCfg, GateCfg, true>(dx_params(dY, W, ldw, dX, M, N, D),
                                                         gate_params(dY, X, cg, partials, M, N, D), device_cus(),
                                                         tail_ws, s);
-    return launch_gemm_dual<DxCfg, GateCfg>(dx_params(dY, W, ldw, dX, M, N, D),
+    return launch_st_dual<DxCfg, GateCfg, false>(dx_params(dY, W, ldw, dX, M, N, D),
                                             gate_params(dY, X, cg, partials, M, N, D), device_cus(), tail_ws, s);
 }
 
 // PTQR forward: token rows grouped by candidate, each group multiplied by its
 // candidate's bf16 decode (the mainloop and store of the forward product, with
 // A rows gathered and Y rows scattered through perm).
-// SWITCH_LOOSE: 1.1-2.2% faster than SWITCH_READ_FIRST at 8192 tokens over six
-// candidates (5120 -> 17408, 4096 -> 28672, 1024 -> 6144)
-using RoutedCfg = GemmCfg<DmaKSG<256, 64, 64 * kWaves>, FwdLB, 256, 256, 64, 4, 2, EPI_STORE, 2, SWITCH_LOOSE, 2, COPY_SPLIT>;
-
 hipError_t launch_routed_fwd(const bf16_t* X, int M, int D, const bf16_t* const* cand_bf16, int64_t ldw, int N,
                              int ncand, const int* perm, const int* group_off, bf16_t* Y, hipStream_t s) {
     GemmParams p = fwd_params(X, nullptr, ldw, Y, M, N, D);
@@ -248,7 +225,7 @@ hipError_t launch_routed_fwd(const bf16_t* X, int M, int D, const bf16_t* const*
     p.ngroups = ncand;
     p.map_rows = M;
     for (int k = 0; k < ncand; ++k) p.bk[k] = cand_bf16[k];
-    return launch_routed_gemm<RoutedCfg>(p, M, device_cus(), s);
+    return launch_st_routed(p, M, device_cus(), s);
 }
 
 // Fixed-order fp64 sum of the work-item partials: dprobs[k] = sum_t partials[t * stride + k].

@@ -1,25 +1,15 @@
-// bf16 MFMA GEMM machinery of the gated Linear on gfx950
-// (v_mfma_f32_32x32x16_bf16).  Included by vq_gemm.hip, which instantiates
-// the tile configurations.
-//
-// One kernel template computes C[i][j] = sum_k A[i][k] * B[j][k] with both
-// operands copied global -> LDS by direct-to-LDS buffer loads into XOR-
-// swizzled stages, then read as MFMA fragments (each lane holds 8
-// consecutive k of one row):
+// bf16 MFMA pieces of the gated Linear on gfx950 shared by the products
+// (v_mfma_f32_32x32x16_bf16 tiles of 128x128 here; the 256x256 products are in
+// vq_gemm_stream.h): direct-to-LDS operand loaders, the order in which tiles
+// become work items, and the small-tile store product
+//   C[i][j] = sum_k A[i][k] * B[j][k].
+// Operands are copied global -> LDS by direct-to-LDS buffer loads into XOR-
+// swizzled stages, then read as MFMA fragments (each lane holds 8 consecutive
+// k of one row):
 //   DmaKS - the source has k contiguous (row-major [rows][K]); fragments
 //           with ds_read_b128;
 //   DmaNS - the source is [K][rows] (rows contiguous), kept in that
 //           orientation; fragments with ds_read_b64_tr_b16.
-// The three products of the path:
-//   forward  Y[m][n]  = sum_d X[m][d] W[n][d]        A=X (KS), B=W (KS)
-//   dX       dX[m][d] = sum_n dY[m][n] W[n][d]       A=dY (KS), B=W (NS)
-//   gate     dW[d][n] = sum_m X[m][d] dY[m][n]       A=X (NS), B=dY (NS)
-// The gate product never reaches global memory: its epilogue keeps the fp32
-// tile in the accumulators, stages each candidate's bytes for the tile into
-// LDS (reusing the main-loop buffers) and dots the exactly decoded weights
-// against it, writing one partial per candidate per work item.  <dW, W_k> is linear in dW, so the M reduction may also be split
-// across work items with no dW reduction at all.  A second kernel sums the
-// partials in a fixed order: gate gradients are deterministic.
 //
 // MFMA 32x32x16 operand/result layout (per wave of 64 lanes):
 //   A: lane l holds A[i = l%32][k = 8*(l/32) .. +7]
@@ -71,8 +61,6 @@ typedef __attribute__((address_space(3))) void lds_void_t;
 // per row the stage is 1/9 (BK 64) smaller, and no copy lane writes padding.
 template <int ROWS, int BK, int THREADS>
 struct DmaKS {
-    static constexpr bool kDma = true;
-    static constexpr int kPerm = 0;
     static constexpr int kFragReads = 1;
     static constexpr int CPR = BK / 8;
     static_assert(CPR == 4 || CPR == 8, "BK 32 or 64");
@@ -90,7 +78,7 @@ struct DmaKS {
             return (r ^ (r >> 3)) & 7;
     }
     // tile rows [r0, r0 + ROWS) of src[row * ld + k]
-    __device__ __forceinline__ void init(int64_t ld, int r0, int rows, const int* = nullptr, int = 0) {
+    __device__ __forceinline__ void init(int64_t ld, int r0, int rows) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
@@ -123,16 +111,8 @@ struct DmaKS {
 // multiples of 32); the XOR moves the 4 k-rows' 64-byte blocks onto distinct
 // quarters of 256 bytes (as a 64-byte pad per k-row would).  The read at
 // k + 4 keeps the same XOR.
-// PERM = 1 reorders each 32-row fragment by 4-row granules: MFMA row 4 q + t
-// reads tile row 4 rot(q) + t, rot(q) = 4 (q % 2) + q / 2.  Accumulator
-// element 4 u + t of lane l (MFMA row 8 u + 4 (l / 32) + t) then holds tile
-// row 16 (l / 32) + 4 u + t: each lane's 16 values of a 32x32 block are 16
-// consecutive tile rows.  Each 32-lane half still reads whole 64-byte blocks
-// of the same 4 k-rows, so the reads stay conflict-free.
-template <int ROWS, int BK, int THREADS, int PERM = 0>
+template <int ROWS, int BK, int THREADS>
 struct DmaNS {
-    static constexpr bool kDma = true;
-    static constexpr int kPerm = PERM;
     static constexpr int kFragReads = 2;
     static constexpr int RCH = ROWS / 8;  // chunks per k-row
     static_assert(RCH % 16 == 0, "the XOR of up to 12 stays inside the k-row");
@@ -144,7 +124,7 @@ struct DmaNS {
     int kpos[NI];
 
     // tile rows [r0, r0 + ROWS) of src[k * ld + row]
-    __device__ __forceinline__ void init(int64_t ld, int r0, int rows, const int* = nullptr, int = 0) {
+    __device__ __forceinline__ void init(int64_t ld, int r0, int rows) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
@@ -169,13 +149,12 @@ struct DmaNS {
     // (measured on gfx950), so when lane s addresses
     //     k = kk + 8 (s/32) + (s%16)/4,   row = r + 16 ((s/16)%2) + 4 (s%4)
     // lane l receives rows r + l%32 at k = kk + 8 (l/32) + 0..3: the MFMA layout
-    // (PERM = 1 moves each addressed 4-row granule as described above)
     static __device__ __forceinline__ bf16x8_t read_frag(const u32x4* __restrict__ lds, int row, int ks, int lane) {
         typedef short v4i16 __attribute__((ext_vector_type(4)));
         typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
         const int k = 16 * ks + 8 * (lane >> 5) + ((lane & 15) >> 2);
         const int q = 4 * ((lane >> 4) & 1) + (lane & 3);  // 4-row granule of the MFMA rows
-        const int r = row + 4 * (PERM ? (((q & 1) << 2) | (q >> 1)) : q);
+        const int r = row + 4 * q;
         const bf16_t* base =
             reinterpret_cast<const bf16_t*>(lds) + 8 * (k * RCH + ((r >> 3) ^ (4 * (k & 3)))) + (r & 7);
         const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(base));
@@ -183,40 +162,6 @@ struct DmaNS {
         typedef short v8i16 __attribute__((ext_vector_type(8)));
         const v8i16 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         return __builtin_bit_cast(bf16x8_t, v);
-    }
-};
-
-// DmaKS with gathered rows: tile row r is source row map[r0 + r] (rows
-// r0 + r >= rows are zeros).  The per-lane offsets carry the whole row offset,
-// so the descriptor base moves with k only; the host bounds m * ld * 2 < 2^31.
-template <int ROWS, int BK, int THREADS>
-struct DmaKSG : DmaKS<ROWS, BK, THREADS> {
-    using Base = DmaKS<ROWS, BK, THREADS>;
-    using Base::CPR;
-    using Base::NI;
-    using Base::NW;
-    // map_rows: valid source rows; an entry outside [0, map_rows) reads zeros
-    __device__ __forceinline__ void init(int64_t ld, int r0, int rows, const int* map, int map_rows) {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int L = (i * NW + wave) * 64 + lane;
-            const int row = L / CPR;
-            const int c = (L % CPR) ^ Base::sw(row);
-            const int src = r0 + row < rows ? map[r0 + row] : -1;
-            const bool ok = (unsigned)src < (unsigned)map_rows;
-            this->voff[i] = ok ? (uint32_t)(((int64_t)src * ld + 8 * c) * 2) : kOOB;
-            this->kpos[i] = 8 * c + 8;
-        }
-    }
-    __device__ __forceinline__ void issue(u32x4* lds, const bf16_t* __restrict__ src, int64_t, int, int k0,
-                                          int kvalid) const {
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc(src + k0);
-        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t*)(lds + (i * NW + wave) * 64), 16,
-                                                     this->kpos[i] <= kvalid ? this->voff[i] : kOOB, 0, 0, 0);
     }
 };
 
@@ -307,10 +252,11 @@ __device__ __forceinline__ WorkItem map_work(int w, int tiles_m, int tiles_n, in
     return wi;
 }
 
-// EPI_STORE: C rounded to bf16.  EPI_GATE: the tile's dots with every
-// candidate (partials per block).  EPI_PARTS: a gate product whose tiles are
-// split along K into p.parts parts writes each part's fp32 tile to p.dwp and
-// leaves the candidate dots to one pass over the summed parts.
+// What becomes of a finished tile.  EPI_STORE: C rounded to bf16.  EPI_GATE: the
+// tile's dots with every candidate (partials per block).  EPI_PARTS: a gate
+// product whose tiles are split along K into p.parts parts writes each part's
+// fp32 tile to p.dwp and leaves the candidate dots to one pass over the summed
+// parts.
 enum Epi : int { EPI_STORE = 0, EPI_GATE = 1, EPI_PARTS = 2 };
 
 struct GemmParams {
@@ -337,13 +283,13 @@ struct GemmParams {
     // parts epilogue: [tile (tm * tiles_j + tn)][part][BJ][BI] fp32, n-major
     float* dwp;
     int parts;
-    // routed product: A rows gathered and C rows scattered through rowmap;
+    // routed product: activation and C rows gathered and scattered through rowmap;
     // group g owns rowmap[group_off[g] .. group_off[g + 1]) and multiplies
     // by bk[g]
     const int* rowmap;
     const int* group_off;
     int ngroups;
-    int map_rows;  // rows of A and C (entries of rowmap outside [0, map_rows) are skipped)
+    int map_rows;  // activation and C rows (entries of rowmap outside [0, map_rows) are skipped)
     const bf16_t* bk[kMaxCand];
 };
 
@@ -360,10 +306,6 @@ struct StageLds {
     static constexpr size_t BYTES = (size_t)DEPTH * (A_CH + B_CH) * 16;  // DEPTH stages
 };
 
-// Main loop with direct-to-LDS loaders and NS LDS stages: the loads of stage
-// kt + NS - 1 are issued right after the barrier that retires stage kt - 1,
-// so NS - 1 stages are in flight while stage kt is multiplied.  One barrier
-// per stage; each wave waits (vmcnt) only for its own copies of stage kt.
 // Wait until at most N of this wave's vector-memory operations are pending,
 // then for its LDS operations, then for the other waves.  A plain
 // __syncthreads() would also drain vmcnt (its release fence), retiring the
@@ -374,47 +316,25 @@ __device__ __forceinline__ void wait_vmcnt_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// Main loop over direct-to-LDS stages: NS LDS stages, NS - 1 of them in
-// flight while one is multiplied.  The stage switch sits inside the MFMA
+// Main loop over direct-to-LDS stages, two in LDS: one in flight while the
+// other is multiplied.  The stage switch sits inside the MFMA
 // stream: the wait for stage kt + 1 and the barrier come after the last
 // k-step's fragments of stage kt are in registers, so the next stage's first
-// fragment reads and the copies of stage kt + NS (into the buffer stage kt just
+// fragment reads and the copies of stage kt + 2 (into the buffer stage kt just
 // vacated) are issued among the last k-step's MFMAs instead of in front of an
 // idle matrix pipe.  Each wave waits (vmcnt) only for its own copies; the
 // barrier then covers everyone's.
-// Order of the stage switch, measured per product on MI355X (operand layout
-// and tile count change which one keeps the matrix pipe busiest):
-//   SWITCH_COPY_FIRST   copies of stage kt + NS, then reads of stage kt + 1
-//   SWITCH_READ_FIRST   reads first, so the copies can interleave the MFMAs
-//   SWITCH_FENCED       reads first, and the barrier fenced with
-//                       sched_barrier so no MFMA or read crosses it
-//   SWITCH_LOOSE        reads first; inside a stage only "the first k-step's
-//                       reads, then its MFMAs" is pinned, the rest is left to
-//                       the scheduler
-//   SWITCH_LOOSE2       SWITCH_LOOSE with the stage switch unpinned too
-//   SWITCH_FREE         no scheduling hints at all (order of issue only)
-enum StageSwitch : int {
-    SWITCH_COPY_FIRST = 0,
-    SWITCH_READ_FIRST = 1,
-    SWITCH_FENCED = 2,
-    SWITCH_LOOSE = 3,
-    SWITCH_LOOSE2 = 4,
-    SWITCH_FREE = 5
-};
-
-// COPY_SPLIT: the refill of the buffer a stage switch frees is issued in two
-// halves, the A tile at the switch and the B tile after the next stage's first
-// k-step, so the two bursts of LDS writes land apart (two stages only: every
-// switch then waits for all copies).
-enum CopyIssue : int { COPY_BURST = 0, COPY_SPLIT = 1 };
-
-template <class LA, class LB, int BI, int BJ, int BK, int WI, int WJ, int NS, int SWITCH, int COPY = COPY_BURST>
+// The refill of the buffer a stage switch frees is issued in two halves, the A
+// tile at the switch and the B tile after the next stage's first k-step, so the
+// two bursts of LDS writes land apart (every switch waits for all copies).
+// After a switch the reads come first: the compiler cannot tell the stage
+// buffers apart, so copies issued first would stay ahead of every later read
+// (and MFMA).
+template <class LA, class LB, int BI, int BJ, int BK, int WI, int WJ>
 __device__ __forceinline__ void gemm_mainloop_pp(const GemmParams& p, int i0, int j0, int kbeg, int kend,
                                                  u32x4* __restrict__ smem,
                                                  f32x16 (&acc)[GemmShape<BI, BJ, BK, WI, WJ>::MI]
                                                               [GemmShape<BI, BJ, BK, WI, WJ>::NJ]) {
-    static_assert(NS >= 2 && NS <= 4, "2 to 4 LDS stages");
-    static_assert(COPY == COPY_BURST || NS == 2, "split refills need the wait-for-all of two stages");
     using S = GemmShape<BI, BJ, BK, WI, WJ>;
     constexpr int STAGE = LA::CHUNKS + LB::CHUNKS;
     constexpr int KS = BK / 16;
@@ -426,7 +346,7 @@ __device__ __forceinline__ void gemm_mainloop_pp(const GemmParams& p, int i0, in
     const int wi = wave / WJ, wj = wave % WJ;
     LA la;
     LB lb;
-    la.init(p.lda, i0, p.I, p.rowmap, p.map_rows);
+    la.init(p.lda, i0, p.I);
     lb.init(p.ldb, j0, p.J);
 #pragma unroll
     for (int a = 0; a < S::MI; ++a)
@@ -437,22 +357,13 @@ __device__ __forceinline__ void gemm_mainloop_pp(const GemmParams& p, int i0, in
 
     const int nk = (kend - kbeg + BK - 1) / BK;
     // stage kt past the end copies nothing (zeros into a free buffer)
-    auto issue = [&](int kt) {
-        u32x4* st = smem + (kt % NS) * STAGE;
-        const int k0 = min(kbeg + kt * BK, kend);
-        const int kvalid = min(BK, kend - k0);
-        la.issue(st, p.A, p.lda, i0, k0, kvalid);
-        lb.issue(st + LA::CHUNKS, p.B, p.ldb, j0, k0, kvalid);
-    };
     auto issue_a = [&](int kt) {
-        u32x4* st = smem + (kt % NS) * STAGE;
         const int k0 = min(kbeg + kt * BK, kend);
-        la.issue(st, p.A, p.lda, i0, k0, min(BK, kend - k0));
+        la.issue(smem + (kt % 2) * STAGE, p.A, p.lda, i0, k0, min(BK, kend - k0));
     };
     auto issue_b = [&](int kt) {
-        u32x4* st = smem + (kt % NS) * STAGE;
         const int k0 = min(kbeg + kt * BK, kend);
-        lb.issue(st + LA::CHUNKS, p.B, p.ldb, j0, k0, min(BK, kend - k0));
+        lb.issue(smem + (kt % 2) * STAGE + LA::CHUNKS, p.B, p.ldb, j0, k0, min(BK, kend - k0));
     };
     bf16x8_t fa[2][S::MI], fb[2][S::NJ];
     auto read = [&](const u32x4* st, int ks, int buf) {
@@ -471,61 +382,42 @@ __device__ __forceinline__ void gemm_mainloop_pp(const GemmParams& p, int i0, in
 
     if (nk <= 0) return;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) issue(s);
-    wait_vmcnt_barrier<(NS - 1) * NI>();
+    for (int s = 0; s < 2; ++s) {
+        issue_a(s);
+        issue_b(s);
+    }
+    wait_vmcnt_barrier<NI>();
     read(smem, 0, 0);
     for (int kt = 0; kt < nk; ++kt) {
-        const u32x4* st = smem + (kt % NS) * STAGE;
+        const u32x4* st = smem + (kt % 2) * STAGE;
 #pragma unroll
         for (int ks = 0; ks + 1 < KS; ++ks) {
             read(st, ks + 1, (ks + 1) & 1);
             mfma(ks & 1);
-            // the B half of the refill issued at the last switch
-            if constexpr (COPY == COPY_SPLIT)
-                if (ks == 0 && kt >= 1) issue_b(kt - 1 + NS);
+            if (ks == 0 && kt >= 1) issue_b(kt + 1);  // the B half of the refill issued at the last switch
         }
-        if constexpr (SWITCH != SWITCH_FREE) __builtin_amdgcn_sched_group_barrier(0x100, FR, 0);  // reads of k-step 1 first
-        if constexpr (SWITCH != SWITCH_LOOSE && SWITCH != SWITCH_FREE && SWITCH != SWITCH_LOOSE2) {
+        __builtin_amdgcn_sched_group_barrier(0x100, FR, 0);  // reads of k-step 1 first
 #pragma unroll
-            for (int ks = 1; ks + 1 < KS; ++ks) {
+        for (int ks = 1; ks + 1 < KS; ++ks) {
 #pragma unroll
-                for (int r = 0; r < FR; ++r) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, (MF + FR - 1) / FR, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                }
+            for (int r = 0; r < FR; ++r) {
+                __builtin_amdgcn_sched_group_barrier(0x008, (MF + FR - 1) / FR, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
         }
-        if constexpr (SWITCH != SWITCH_FREE) __builtin_amdgcn_sched_group_barrier(0x008, MF, 0);
-        // all of stage kt is in registers: wait for stage kt + 1 (stages
-        // kt + 2 .. kt + NS - 1 may still be in flight), then stage kt's
-        // buffer is free for stage kt + NS (past the end: harmless zeros and
-        // reads, so the body has no branch and one set of accumulators)
-        // SWITCH_FENCED: the barrier becomes a hard scheduling boundary (the
-        // scheduler otherwise moves register-only MFMAs from above past it and
-        // fragment reads from below ahead of it)
-        if constexpr (SWITCH == SWITCH_FENCED) __builtin_amdgcn_sched_barrier(0);
-        wait_vmcnt_barrier<(NS - 2) * NI>();
-        if constexpr (SWITCH == SWITCH_FENCED) __builtin_amdgcn_sched_barrier(0);
-        // reads first: the compiler cannot tell stage buffers apart, so copies
-        // issued first stay ahead of every later read (and MFMA)
-        if constexpr (COPY == COPY_SPLIT) {
-            read(smem + ((kt + 1) % NS) * STAGE, 0, 0);
-            issue_a(kt + NS);
-        } else if constexpr (SWITCH == SWITCH_COPY_FIRST) {
-            issue(kt + NS);
-            read(smem + ((kt + 1) % NS) * STAGE, 0, 0);
-        } else {
-            read(smem + ((kt + 1) % NS) * STAGE, 0, 0);
-            issue(kt + NS);
-        }
+        __builtin_amdgcn_sched_group_barrier(0x008, MF, 0);
+        // all of stage kt is in registers: wait for stage kt + 1, then stage
+        // kt's buffer is free for stage kt + 2 (past the end: harmless zeros
+        // and reads, so the body has no branch and one set of accumulators)
+        wait_vmcnt_barrier<0>();
+        read(smem + ((kt + 1) % 2) * STAGE, 0, 0);
+        issue_a(kt + 2);
         mfma((KS - 1) & 1);
-        if constexpr (SWITCH != SWITCH_FREE && SWITCH != SWITCH_LOOSE2) {
-            __builtin_amdgcn_sched_group_barrier(0x100, FR, 1);
+        __builtin_amdgcn_sched_group_barrier(0x100, FR, 1);
 #pragma unroll
-            for (int r = 0; r < MF; ++r) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
-                __builtin_amdgcn_sched_group_barrier(0x020, (NI + MF - 1) / MF, 1);
-            }
+        for (int r = 0; r < MF; ++r) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x020, (NI + MF - 1) / MF, 1);
         }
     }
     wait_vmcnt_barrier<0>();  // the zero copies have landed before anyone reuses LDS
@@ -553,192 +445,25 @@ constexpr int kGateMaxChunks = gate_span_chunks(272);  // worst type (Q8_0)
 
 __device__ __forceinline__ int gate_row_chunks(int qt) { return gate_span_chunks(group_bytes(qt)); }
 
-template <int BJ, int THREADS>
-__device__ __forceinline__ void gate_stage_lds(u32x4* __restrict__ buf, const uint8_t* __restrict__ qbytes, int qt,
-                                               int64_t row_groups, int j0, int group, int J) {
-    typedef __attribute__((address_space(3))) void lds_void;
-    const int gb = group_bytes(qt), nch = gate_row_chunks(qt);
-    const int64_t origin = ((int64_t)j0 * row_groups * gb) & ~int64_t(15);
-    const int64_t bytes = (int64_t)J * row_groups * gb - origin;
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(qbytes + origin), (short)0, (int)(bytes < (int64_t)kRange ? bytes : (int64_t)kRange),
-        0x00020000);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int NW = THREADS / 64;
-    const int total = BJ * nch;
-    for (int base = wave * 64; base < total; base += NW * 64) {
-        const int id = base + lane;
-        const int row = id / nch, c = id % nch;
-        const int n = (j0 + row < J && id < total) ? j0 + row : j0;
-        const int64_t span = ((int64_t)n * row_groups + group) * gb;
-        // one instruction per wave: lanes land at buf + 16 (base + lane)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(buf + base), 16,
-                                                 (uint32_t)((span & ~int64_t(15)) - origin + 16 * c), 0, 0, 0);
-    }
-}
-
-// <acc, W_k> over the lane's accumulators: with the A operand's rows
-// permuted (DmaNS PERM = 1), block (a, b) holds, for row n = 32 b + lane%32,
-// the 16 consecutive weights 32 a + 16 (lane/32) + r, r = 0..15 (relative to
-// the wave's tile origin).
-template <int QT, int MI, int NJ, int WTI, int WTJ>
-__device__ __forceinline__ float gate_dot_lds(const f32x16 (&acc)[MI][NJ], const float (&sv)[MI][NJ],
-                                              const uint8_t* __restrict__ buf, int64_t row_groups, int j0, int group,
-                                              int wi, int wj, int lane, int J) {
-    constexpr int GB = group_bytes(QT);
-    constexpr int PITCH = 16 * gate_span_chunks(GB);  // bytes per staged row span
-    float s = 0.0f;
-#pragma unroll
-    for (int b = 0; b < NJ; ++b) {
-        const int nl = wj * WTJ + 32 * b + (lane & 31);
-        // rows past J were staged from the tile's first row: locate their bytes the same way
-        const int n = j0 + nl < J ? j0 + nl : j0;
-        const int64_t span = ((int64_t)n * row_groups + group) * GB;
-        const uint8_t* g = buf + nl * PITCH + (int)(span & 15);
-#pragma unroll
-        for (int a = 0; a < MI; ++a) {
-            float v[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) v[r] = acc[a][b][r];
-            s += dot_sub16<QT>(g, wi * WTI + 32 * a + 16 * (lane >> 5), v, sv[a][b]);
-        }
-    }
-    return s;
-}
-
-// gate_dot_lds for the IQ formats (type known at run time, uniform)
-template <int MI, int NJ, int WTI, int WTJ>
-__device__ __forceinline__ float gate_dot_lds_iq(int qt, const f32x16 (&acc)[MI][NJ], const float (&sv)[MI][NJ],
-                                                 const uint8_t* __restrict__ buf, int64_t row_groups, int j0,
-                                                 int group, int wi, int wj, int lane, int J) {
-    const int gb = group_bytes(qt);
-    const int pitch = 16 * gate_span_chunks(gb);
-    float s = 0.0f;
-#pragma unroll
-    for (int b = 0; b < NJ; ++b) {
-        const int nl = wj * WTJ + 32 * b + (lane & 31);
-        const int n = j0 + nl < J ? j0 + nl : j0;
-        const int64_t span = ((int64_t)n * row_groups + group) * gb;
-        const uint8_t* g = buf + nl * pitch + (int)(span & 15);
-#pragma unroll
-        for (int a = 0; a < MI; ++a) {
-            float v[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) v[r] = acc[a][b][r];
-            s += dot_sub16_iq(qt, g, wi * WTI + 32 * a + 16 * (lane >> 5), v, sv[a][b]);
-        }
-    }
-    return s;
-}
-
-// IQ: the candidate set may hold IQ formats (their table-lookup decode needs
-// registers the K-quant-only instantiation keeps for itself).
-template <int BI, int BJ, int BK, int WI, int WJ, bool IQ>
-__device__ __forceinline__ void gate_epilogue(const GemmParams& p, int block, int i0, int j0,
-                                              u32x4* __restrict__ smem,
-                                              const f32x16 (&acc)[GemmShape<BI, BJ, BK, WI, WJ>::MI]
-                                                                 [GemmShape<BI, BJ, BK, WI, WJ>::NJ]) {
-    using S = GemmShape<BI, BJ, BK, WI, WJ>;
-    static_assert(BI == 256, "the gate tile covers exactly one 256-weight group per row");
-    constexpr int NW = WI * WJ;
-    constexpr int BUF_CH = BJ * kGateMaxChunks;  // 16-byte chunks per candidate buffer
-    // per-wave candidate sums, after the two candidate buffers (inside the
-    // dynamic allocation: a static array would push an 8-wave workgroup whose
-    // main loop takes all 160 KiB past the limit)
-    float(*red)[kMaxCand] = reinterpret_cast<float(*)[kMaxCand]>(smem + 2 * BUF_CH);
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scale fields index by it
-    const int wi = wave / WJ, wj = wave % WJ;
-    const int group = i0 / 256;
-    // the gated tensor this tile's rows belong to (uniform per block)
-    int g = 0;
-#pragma unroll
-    for (int q = 1; q < kMaxSets; ++q)
-        if (q < p.cg.nsets && j0 >= p.cg.set_j0[q]) g = q;
-    const CandSet& cs = p.cg.sets[g];
-    const int jl0 = j0 - p.cg.set_j0[g];                 // first row within the tensor
-    const int jn = p.cg.set_j0[g + 1] - p.cg.set_j0[g];  // the tensor's rows
-    const int64_t rg = cs.row_groups;
-    // candidate-independent sums of each accumulator block
-    float sv[S::MI][S::NJ];
-#pragma unroll
-    for (int a = 0; a < S::MI; ++a)
-#pragma unroll
-        for (int b = 0; b < S::NJ; ++b) {
-            float t = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) t += acc[a][b][r];
-            sv[a][b] = t;
-        }
-    __syncthreads();  // every wave is past its last main-loop LDS read
-    gate_stage_lds<BJ, S::THREADS>(smem, cs.qbytes[0], cs.qtype[0], rg, jl0, group, jn);
-    for (int k = 0; k < cs.ncand; ++k) {
-        // this wave's direct-to-LDS copies of candidate k have landed, then
-        // everyone's have; buffer (k+1) % 2 is no longer read
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (k + 1 < cs.ncand)
-            gate_stage_lds<BJ, S::THREADS>(smem + ((k + 1) & 1) * BUF_CH, cs.qbytes[k + 1], cs.qtype[k + 1], rg, jl0,
-                                           group, jn);
-        const uint8_t* buf = reinterpret_cast<const uint8_t*>(smem + (k & 1) * BUF_CH);
-        float sum;
-        switch (cs.qtype[k]) {
-        case Q8_0: sum = gate_dot_lds<Q8_0, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wi, wj, lane, jn); break;
-        case Q2_K: sum = gate_dot_lds<Q2_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wi, wj, lane, jn); break;
-        case Q3_K: sum = gate_dot_lds<Q3_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wi, wj, lane, jn); break;
-        case Q4_K: sum = gate_dot_lds<Q4_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wi, wj, lane, jn); break;
-        case Q5_K: sum = gate_dot_lds<Q5_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wi, wj, lane, jn); break;
-        default:
-            if constexpr (IQ) {
-                if (is_iq(cs.qtype[k])) {
-                    sum = gate_dot_lds_iq<S::MI, S::NJ, S::WTI, S::WTJ>(cs.qtype[k], acc, sv, buf, rg, jl0, group, wi,
-                                                                        wj, lane, jn);
-                    break;
-                }
-            }
-            sum = gate_dot_lds<Q6_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wi, wj, lane, jn);
-            break;
-        }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
-        if (lane == 0) red[wave][k] = sum;
-    }
-    __syncthreads();
-    // this block's slots of every tensor: its own sums, zeros for the others
-    const int nslot = p.cg.nsets * p.cg.kstride;
-    if ((int)threadIdx.x < nslot) {
-        const int k = (int)threadIdx.x - g * p.cg.kstride;
-        float s = 0.0f;
-        if (k >= 0 && k < cs.ncand)
-            for (int wv = 0; wv < NW; ++wv) s += red[wv][k];
-        p.partials[(int64_t)block * nslot + threadIdx.x] = s;
-    }
-}
-
 // ---------------------------------------------------------------- kernels
-// One GEMM configuration: loaders, tile, wave layout, epilogue, pipeline depth.
 // K steps a split part of a store tile must save (see GemmCfg::plan).  14
 // against 10: the dual backward at 8192 tokens, 1024 -> 1536 (24 K steps of
 // dX, no longer split in two) 94 -> 82 us; within 0.5% at 5120 -> 17408,
 // 4096 -> 28672 and the other 1024-wide products.
 constexpr int kMinSavedSplitSteps = 14;
 
-template <class LA_, class LB_, int BI_, int BJ_, int BK_, int WI_, int WJ_, int EPI_, int DEPTH_,
-          int SWITCH_ = SWITCH_FENCED, int OCC_ = 1, int COPY_ = COPY_BURST>
+// One small-tile configuration: loaders, tile, wave layout.
+template <class LA_, class LB_, int BI_, int BJ_, int BK_, int WI_, int WJ_, int OCC_>
 struct GemmCfg {
     using LA = LA_;
     using LB = LB_;
-    static constexpr int BI = BI_, BJ = BJ_, BK = BK_, WI = WI_, WJ = WJ_, EPI = EPI_, DEPTH = DEPTH_;
-    static constexpr int SWITCH = SWITCH_;
+    static constexpr int BI = BI_, BJ = BJ_, BK = BK_, WI = WI_, WJ = WJ_;
     static constexpr int OCC = OCC_;  // waves per SIMD the registers are budgeted for
-    static constexpr int COPY = COPY_;
     static constexpr int THREADS = WI * WJ * 64;
-    static constexpr size_t main_lds() { return StageLds<LA, LB, DEPTH>::BYTES; }
     static constexpr size_t lds() {
-        constexpr size_t gate = (size_t)2 * BJ * kGateMaxChunks * 16 + (size_t)WI * WJ * kMaxCand * 4;  // two candidate buffers, wave sums
-        constexpr size_t store = (size_t)BI * (BJ + 8) * 2 + BI * 4;   // bf16 staging of the tile, row map
-        constexpr size_t epi = EPI == EPI_GATE ? gate : EPI == EPI_PARTS ? 0 : store;
-        return epi > main_lds() ? epi : main_lds();
+        constexpr size_t store = (size_t)BI * (BJ + 8) * 2;  // bf16 staging of the tile
+        constexpr size_t main = StageLds<LA, LB, 2>::BYTES;
+        return store > main ? store : main;
     }
     static int tiles_i(const GemmParams& p) { return (p.I + BI - 1) / BI; }
     static int tiles_j(const GemmParams& p) { return (p.J + BJ - 1) / BJ; }
@@ -746,25 +471,9 @@ struct GemmCfg {
     // Fill in the work decomposition; returns the grid size (8 * blocks per XCD).
     static int plan(GemmParams& p, int cus, bool split_ok) {
         if (p.I <= 0 || p.J <= 0) return 0;
-        if constexpr (EPI == EPI_PARTS) {
-            // every tile in p.parts parts, the XCDs' tile ranges as for whole tiles
-            p.cus_per_xcd = cus / 8 > 0 ? cus / 8 : 1;
-            p.split_ok = 0;
-            p.tail_max = 0;
-            p.s_max = 1;
-            const int tiles = tiles_i(p) * tiles_j(p);
-            int items = 0;
-            for (int x = 0; x < 8; ++x) {
-                const XcdPlan pl = xcd_plan(x, tiles, p.cus_per_xcd, ksteps(p), false);
-                items = pl.tiles * p.parts > items ? pl.tiles * p.parts : items;
-            }
-            return 8 * items;
-        }
         // a split store tile pays for its partial writes and a fixup launch:
         // split only when a part saves at least kMinSavedSplitSteps K steps
-        p.split_min_saved = EPI == EPI_STORE ? kMinSavedSplitSteps : 0;
-        // more than 8 parts (tried for the gate at 1024 x 1024) loses: the
-        // parts of a dual launch then overflow one round of the CUs
+        p.split_min_saved = kMinSavedSplitSteps;
         p.split_max = 8;
         p.cus_per_xcd = cus / 8 > 0 ? cus / 8 : 1;
         p.split_ok = split_ok ? 1 : 0;
@@ -780,7 +489,7 @@ struct GemmCfg {
         }
         return 8 * items;
     }
-    // fp32 workspace the split tails of a store epilogue need
+    // fp32 workspace the split tails need
     static int64_t tail_bytes(const GemmParams& p) {
         return p.tail_max > 0 ? (int64_t)8 * p.tail_max * p.s_max * BI * BJ * 4 : 0;
     }
@@ -799,18 +508,11 @@ __device__ __forceinline__ void store_tile_lds(const GemmParams& p, int i0, int 
                                                                   [GemmShape<BI, BJ, BK, WI, WJ>::NJ]) {
     using S = GemmShape<BI, BJ, BK, WI, WJ>;
     constexpr int PITCH = BJ + 8;  // bf16 per LDS row
-    static_assert((size_t)BI * PITCH * 2 + BI * 4 <= 160 * 1024, "tile and row map fit in LDS");
-    static_assert(S::THREADS >= BI, "one thread per tile row loads the row map");
+    static_assert((size_t)BI * PITCH * 2 <= 160 * 1024, "the tile fits in LDS");
     bf16_t* t = reinterpret_cast<bf16_t*>(smem);
-    int* rows_at = reinterpret_cast<int*>(t + BI * PITCH);  // routed: the tile's destination rows
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wi = wave / WJ, wj = wave % WJ;
-    // one map load per tile row, in flight while the accumulators go to LDS
-    // (the store loop below would otherwise wait on a global load per chunk)
-    int dest = -1;
-    if (p.rowmap && (int)threadIdx.x < BI && i0 + (int)threadIdx.x < p.I) dest = p.rowmap[i0 + threadIdx.x];
     __syncthreads();  // every wave is past its last main-loop LDS read
-    if (p.rowmap && (int)threadIdx.x < BI) rows_at[threadIdx.x] = dest;
     // rows il and il + 1 of a lane's column convert as one pair
     // (v_cvt_pk_bf16_f32: one instruction for two values, where the software
     // rounding takes six per value; a NaN stays a quiet NaN)
@@ -835,65 +537,23 @@ __device__ __forceinline__ void store_tile_lds(const GemmParams& p, int i0, int 
         const int il = c / CPR, jc = c % CPR;
         if (il < rows && 8 * jc < cols) {
             const u32x4 v = *reinterpret_cast<const u32x4*>(t + il * PITCH + 8 * jc);
-            const int64_t gi = p.rowmap ? rows_at[il] : i0 + il;  // routed: scatter rows
-            if (!p.rowmap || (uint64_t)gi < (uint64_t)p.map_rows)
-                __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p.C + gi * p.ldc + j0 + 8 * jc));
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p.C + (int64_t)(i0 + il) * p.ldc + j0 + 8 * jc));
         }
     }
 }
 
-// Work item `block` of problem p.  IQ: a gate product whose candidate sets
-// may hold IQ formats (their table-lookup decode needs registers the
-// K-quant-only instantiation keeps for itself).
-template <class C, bool IQ = false>
+// Work item `block` of problem p.
+template <class C>
 __device__ __forceinline__ void gemm_body(const GemmParams& p, int block, u32x4* __restrict__ smem) {
     using LA = typename C::LA;
     using LB = typename C::LB;
-    constexpr int BI = C::BI, BJ = C::BJ, BK = C::BK, WI = C::WI, WJ = C::WJ, EPI = C::EPI, DEPTH = C::DEPTH;
+    constexpr int BI = C::BI, BJ = C::BJ, BK = C::BK, WI = C::WI, WJ = C::WJ;
     using S = GemmShape<BI, BJ, BK, WI, WJ>;
     const int tiles_i = (p.I + BI - 1) / BI, tiles_j = (p.J + BJ - 1) / BJ;
     const int ksteps = (p.K + BK - 1) / BK;
-    if constexpr (EPI == EPI_PARTS) {
-        // item (tile, part): XCD x = block % 8 takes its tile range part by part
-        static_assert(LA::kPerm == 1, "each lane holds 16 consecutive rows i of an accumulator block");
-        const int x = block % 8, local = block / 8;
-        const XcdPlan pl = xcd_plan(x, tiles_i * tiles_j, p.cus_per_xcd, ksteps, false);
-        if (local >= pl.tiles * p.parts) return;
-        int tm, tn;
-        tile_coords(pl.t0 + local / p.parts, tiles_i, tiles_j, kGroupM, tm, tn);
-        const int part = local % p.parts;
-        const int chunk = (ksteps + p.parts - 1) / p.parts * BK;
-        const int kbeg = min(p.K, part * chunk), kend = min(p.K, kbeg + chunk);
-        f32x16 acc[S::MI][S::NJ];
-        gemm_mainloop_pp<LA, LB, BI, BJ, BK, WI, WJ, DEPTH, C::SWITCH, C::COPY>(p, tm * BI, tn * BJ, kbeg, kend, smem,
-                                                                                acc);
-        // acc[a][b][r] is element (i, j) = (wi WTI + 32 a + 16 (lane >> 5) + r, wj WTJ + 32 b + lane % 32):
-        // four 16-byte stores per lane and block, two lanes per 128-byte row segment
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int wi = wave / WJ, wj = wave % WJ;
-        float* slot = p.dwp + ((int64_t)(tm * tiles_j + tn) * p.parts + part) * (BI * BJ);
-#pragma unroll
-        for (int a = 0; a < S::MI; ++a)
-#pragma unroll
-            for (int b = 0; b < S::NJ; ++b) {
-                const int jl = wj * S::WTJ + 32 * b + (lane & 31);
-                const int il = wi * S::WTI + 32 * a + 16 * (lane >> 5);
-                float4* o = reinterpret_cast<float4*>(slot + jl * BI + il);
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    o[q] = make_float4(acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]);
-            }
-        return;
-    }
     const WorkItem w = map_work(block, tiles_i, tiles_j, ksteps, p.cus_per_xcd, p.split_ok != 0, p.tail_max, kGroupM,
                                 p.split_min_saved, p.split_max);
-    if (w.idle) {
-        if constexpr (EPI == EPI_GATE) {
-            const int nslot = p.cg.nsets * p.cg.kstride;
-            if ((int)threadIdx.x < nslot) p.partials[(int64_t)block * nslot + threadIdx.x] = 0.0f;
-        }
-        return;
-    }
+    if (w.idle) return;
     const int i0 = w.tm * BI, j0 = w.tn * BJ;
     int kbeg = 0, kend = p.K;
     if (w.ns > 1) {
@@ -902,27 +562,19 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p, int block, u32x4*
         kend = min(p.K, kbeg + chunk);
     }
     f32x16 acc[S::MI][S::NJ];
-    static_assert(LA::kDma && LB::kDma, "direct-to-LDS loaders");
-    gemm_mainloop_pp<LA, LB, BI, BJ, BK, WI, WJ, DEPTH, C::SWITCH, C::COPY>(p, i0, j0, kbeg, kend, smem, acc);
-
-    if constexpr (EPI == EPI_STORE) {
-        if (w.ns > 1) {
-            // K part of a split tail tile: fp32 partial, [element][thread]
-            float* slot = p.partials + ((int64_t)w.tail_slot * p.s_max + w.split) * (BI * BJ);
+    gemm_mainloop_pp<LA, LB, BI, BJ, BK, WI, WJ>(p, i0, j0, kbeg, kend, smem, acc);
+    if (w.ns > 1) {
+        // K part of a split tail tile: fp32 partial, [element][thread]
+        float* slot = p.partials + ((int64_t)w.tail_slot * p.s_max + w.split) * (BI * BJ);
 #pragma unroll
-            for (int a = 0; a < S::MI; ++a)
+        for (int a = 0; a < S::MI; ++a)
 #pragma unroll
-                for (int b = 0; b < S::NJ; ++b)
+            for (int b = 0; b < S::NJ; ++b)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        slot[((a * S::NJ + b) * 16 + r) * S::THREADS + threadIdx.x] = acc[a][b][r];
-            return;
-        }
-        store_tile_lds<BI, BJ, BK, WI, WJ>(p, i0, j0, smem, acc);
-    } else if constexpr (EPI == EPI_GATE) {
-        static_assert(LA::kPerm == 1, "the gate epilogue reads 16 consecutive weights per accumulator block");
-        gate_epilogue<BI, BJ, BK, WI, WJ, IQ>(p, block, i0, j0, smem, acc);
+                for (int r = 0; r < 16; ++r) slot[((a * S::NJ + b) * 16 + r) * S::THREADS + threadIdx.x] = acc[a][b][r];
+        return;
     }
+    store_tile_lds<BI, BJ, BK, WI, WJ>(p, i0, j0, smem, acc);
 }
 
 // Sum of the K parts of each split tail tile of a store epilogue, in part
@@ -967,41 +619,15 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tail_fixup_kernel(GemmParams 
 }
 
 // The register budget is set by the waves per SIMD the configuration runs at
-// (OCC: one for four-wave 256x256 tiles with 256 accumulators per lane, two
-// for eight-wave ones or two 128x128 workgroups per CU): telling the compiler
+// (OCC: two, for two 128x128 workgroups per CU): telling the compiler
 // so lets it keep fragments in flight instead of minimising registers for an
 // occupancy the LDS use rules out anyway.
-template <class C, bool IQ = false>
+template <class C>
 __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(C::OCC, C::OCC)))
 void gemm_kernel(GemmParams p) {
-#if defined(__HIP_DEVICE_COMPILE__)  // the host pass needs only the launch stub (see gemm_dual_kernel)
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass needs only the launch stub
     extern __shared__ u32x4 smem[];
-    gemm_body<C, IQ>(p, blockIdx.x, smem);
-#endif
-}
-
-// Two independent products in one launch: blocks [0, n1) run problem 1,
-// blocks [n1, ...) problem 2 (n1 is a multiple of 8, so both keep the XCD
-// mapping of map_work; blocks past problem 1's items exit).  One grid lets
-// the second product's work items fill the last, partial round of the first
-// instead of each launch idling CUs in its own tail.
-template <class C1, class C2, bool IQ1 = false, bool IQ2 = false>
-__global__ __launch_bounds__(C1::THREADS) __attribute__((amdgpu_waves_per_eu(C1::OCC, C1::OCC)))
-void gemm_dual_kernel(GemmParams p1, int items1, int n1, GemmParams p2) {
-    static_assert(C1::THREADS == C2::THREADS && C1::OCC == C2::OCC, "both problems use the same workgroup shape");
-    // Kernel bodies are compiled for the device only: the host pass needs just
-    // the launch stub, and with a configuration instantiated for both IQ
-    // values it rejects the second instantiation of gemm_mainloop_pp
-    // (a substitution failure on the accumulator array parameter that the
-    // device pass does not report).
-#if defined(__HIP_DEVICE_COMPILE__)
-    extern __shared__ u32x4 smem[];
-    const int b = blockIdx.x;
-    if (b < n1) {
-        if (b < items1) gemm_body<C1, IQ1>(p1, b, smem);
-    } else {
-        gemm_body<C2, IQ2>(p2, b - n1, smem);
-    }
+    gemm_body<C>(p, blockIdx.x, smem);
 #endif
 }
 
@@ -1016,133 +642,24 @@ static hipError_t set_lds_attr(const void* kern, size_t lds, bool& done) {
     return e;
 }
 
-// Launch of one product.  `cus` is the device's CU count; a store epilogue
-// splits tail tiles only when `tail_ws` (tail_bytes of the plan) is given.
-template <class C, bool IQ = false>
+// Launch of one product.  `cus` is the device's CU count; tail tiles are split
+// only when `tail_ws` (tail_bytes of the plan) is given.
+template <class C>
 static hipError_t launch_gemm_cfg(GemmParams p, int cus, float* tail_ws, hipStream_t s) {
-    const bool split_ok = C::EPI == EPI_GATE || tail_ws != nullptr;
-    const int grid = C::plan(p, cus, split_ok);
+    const int grid = C::plan(p, cus, tail_ws != nullptr);
     if (grid == 0) return hipSuccess;
-    if (C::EPI == EPI_STORE) p.partials = tail_ws;
+    p.partials = tail_ws;
     constexpr size_t lds = C::lds();
     static_assert(lds <= 160 * 1024, "exceeds the 160 KiB of LDS per workgroup");
     static bool attr_set = false;  // per instantiation
-    auto kern = gemm_kernel<C, IQ>;
+    auto kern = gemm_kernel<C>;
     hipError_t e = set_lds_attr<C>((const void*)kern, lds, attr_set);
     if (e != hipSuccess) return e;
     kern<<<dim3(grid), dim3(C::THREADS), lds, s>>>(p);
     e = hipGetLastError();
-    if (e != hipSuccess || C::EPI != EPI_STORE || p.tail_max == 0) return e;
+    if (e != hipSuccess || p.tail_max == 0) return e;
     constexpr int FIX_BLOCKS = GemmShape<C::BI, C::BJ, C::BK, C::WI, C::WJ>::MI * GemmShape<C::BI, C::BJ, C::BK, C::WI, C::WJ>::NJ;
     gemm_tail_fixup_kernel<C><<<dim3(8 * p.tail_max * FIX_BLOCKS), dim3(C::THREADS), 0, s>>>(p);
-    return hipGetLastError();
-}
-
-// Two products in one launch (see gemm_dual_kernel): problem 1, a store
-// product with split tails (tail_ws1), and problem 2, a gate product.  The
-// gate product's work items come first and the store product's fill the
-// tail (its split parts are fixed up after the launch): 0.8-1.5% faster than
-// the other order at 8192 tokens and 5120 -> 17408, 0.9-1.2% at
-// 4096 -> 28672, neutral at 17408 -> 5120 and the 1024-wide products.
-template <class C1, class C2, bool IQ2 = false>
-static hipError_t launch_gemm_dual(GemmParams p1, GemmParams p2, int cus, float* tail_ws1, hipStream_t s) {
-    static_assert(C1::EPI == EPI_STORE && (C2::EPI == EPI_GATE || C2::EPI == EPI_PARTS),
-                  "a store product and a gate product");
-    const int grid1 = C1::plan(p1, cus, tail_ws1 != nullptr);
-    const int grid2 = C2::plan(p2, cus, true);
-    p1.partials = tail_ws1;
-    if (grid1 == 0) return launch_gemm_cfg<C2, IQ2>(p2, cus, nullptr, s);
-    if (grid2 == 0) return launch_gemm_cfg<C1>(p1, cus, tail_ws1, s);
-    constexpr size_t lds = C1::lds() > C2::lds() ? C1::lds() : C2::lds();
-    static_assert(lds <= 160 * 1024, "exceeds the 160 KiB of LDS per workgroup");
-    static bool attr_set = false;
-    auto kern = gemm_dual_kernel<C2, C1, IQ2, false>;
-    hipError_t e = set_lds_attr<C2>((const void*)kern, lds, attr_set);
-    if (e != hipSuccess) return e;
-    kern<<<dim3(grid2 + grid1), dim3(C2::THREADS), lds, s>>>(p2, grid2, grid2, p1);
-    e = hipGetLastError();
-    if (e != hipSuccess || C1::EPI != EPI_STORE || p1.tail_max == 0) return e;
-    constexpr int FIX_BLOCKS = GemmShape<C1::BI, C1::BJ, C1::BK, C1::WI, C1::WJ>::MI * GemmShape<C1::BI, C1::BJ, C1::BK, C1::WI, C1::WJ>::NJ;
-    gemm_tail_fixup_kernel<C1><<<dim3(8 * p1.tail_max * FIX_BLOCKS), dim3(C1::THREADS), 0, s>>>(p1);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------- routed product
-// Grouped GEMM: C[rowmap[r]] = A[rowmap[r]] . bk[g]^T for the rows r of each
-// group g (group_off on the device, so the host never waits for the counts).
-// The grid covers ceil(m / BI) + ngroups - 1 tile-rows, the most the groups can
-// need; every block counts the tile-rows the groups do need, takes its tile of
-// those (the XCDs get even contiguous ranges, the spare blocks spread over all
-// of them) and finds the tile's group by walking the group sizes.  Measured on
-// MI355X at 8192 tokens, 5120 -> 17408, six candidates: group-ordered tiles and
-// the row map staged once per tile took six Gumbel-sized groups from 1.380 to
-// 1.338 ms and six 256-aligned groups from 1.236-1.260 to 1.214 ms (one group
-// 1.145 ms, the dense forward 1.147 ms).
-template <class C>
-__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(C::OCC, C::OCC)))
-void routed_gemm_kernel(GemmParams p, int tile_rows) {
-    using LA = typename C::LA;
-    using LB = typename C::LB;
-    constexpr int BI = C::BI, BJ = C::BJ, BK = C::BK, WI = C::WI, WJ = C::WJ;
-    using S = GemmShape<BI, BJ, BK, WI, WJ>;
-    extern __shared__ u32x4 smem[];
-    const int tiles_j = (p.J + BJ - 1) / BJ;
-    // group bounds clamped to [0, map_rows] and made monotonic, so bad
-    // offsets cannot index rowmap out of range; the work is spread over the
-    // tile-rows the groups actually have (the grid covers the most they can)
-    int used_rows = 0;
-    for (int g = 0, h = 0; g < p.ngroups; ++g) {
-        const int l = min(max(p.group_off[g], h), p.map_rows);
-        h = min(max(p.group_off[g + 1], l), p.map_rows);
-        used_rows += (h - l + BI - 1) / BI;
-    }
-    used_rows = min(used_rows, tile_rows);
-    // the XCDs take contiguous ranges of the tiles (as in map_work); the tiles
-    // run group by group, each group's tile-rows in blocks of kGroupM with the
-    // tile-rows fastest, so the tiles an XCD runs at once read one candidate's
-    // B panels and share them in its L2
-    const int x = blockIdx.x % 8, local = blockIdx.x / 8;
-    const XcdPlan pl = xcd_plan(x, used_rows * tiles_j, p.cus_per_xcd, 0, false);
-    if (local >= pl.items()) return;
-    int tile = pl.t0 + local, tm = 0, tn = 0, g = 0, lo = 0, hi = 0;
-    for (; g < p.ngroups; ++g) {
-        lo = min(max(p.group_off[g], hi), p.map_rows);
-        hi = min(max(p.group_off[g + 1], lo), p.map_rows);
-        const int nt = (hi - lo + BI - 1) / BI;
-        if (tile < nt * tiles_j) {
-            tile_coords(tile, nt, tiles_j, kGroupM, tm, tn);
-            break;
-        }
-        tile -= nt * tiles_j;
-    }
-    if (g >= p.ngroups) return;
-    GemmParams q = p;
-    q.B = p.bk[g];
-    q.I = hi;  // end of the group's rows in rowmap
-    const int i0 = lo + tm * BI, j0 = tn * BJ;
-    f32x16 acc[S::MI][S::NJ];
-    gemm_mainloop_pp<LA, LB, BI, BJ, BK, WI, WJ, C::DEPTH, C::SWITCH, C::COPY>(q, i0, j0, 0, q.K, smem, acc);
-    store_tile_lds<BI, BJ, BK, WI, WJ>(q, i0, j0, smem, acc);
-}
-
-template <class C>
-static hipError_t launch_routed_gemm(GemmParams p, int m, int cus, hipStream_t s) {
-    if (m <= 0 || p.J <= 0 || p.ngroups <= 0) return hipSuccess;
-    const int tile_rows = (m + C::BI - 1) / C::BI + p.ngroups - 1;
-    const int tiles = tile_rows * ((p.J + C::BJ - 1) / C::BJ);
-    p.cus_per_xcd = cus / 8 > 0 ? cus / 8 : 1;
-    p.split_ok = 0;
-    int items = 0;
-    for (int x = 0; x < 8; ++x) {
-        const XcdPlan pl = xcd_plan(x, tiles, p.cus_per_xcd, C::ksteps(p), false);
-        items = pl.items() > items ? pl.items() : items;
-    }
-    constexpr size_t lds = C::lds();
-    static bool attr_set = false;
-    auto kern = routed_gemm_kernel<C>;
-    hipError_t e = set_lds_attr<C>((const void*)kern, lds, attr_set);
-    if (e != hipSuccess) return e;
-    kern<<<dim3(8 * items), dim3(C::THREADS), lds, s>>>(p, tile_rows);
     return hipGetLastError();
 }
 
