@@ -5,7 +5,7 @@
 // F.softmax and F.kl_div over [tokens, vocab] logits, then autograd).
 //
 // Forward: one workgroup per token row streams the student and teacher rows
-// once (16-byte loads) and keeps per-lane online log-sum-exps of s, s/T and
+// once (16-byte loads, the next ones in flight while these are summed) and keeps per-lane online log-sum-exps of s, s/T and
 // t/T, plus A = sum exp(t/T - m_t) (t - s), so that
 //   CE_r = lse(s) - s[y_r]
 //   KL_r = T^2 (A / Z_t / T - lse(t/T) + lse(s/T))     (= T^2 sum p (log p - log q))
@@ -14,9 +14,12 @@
 // the cross-entropy, as F.cross_entropy's default ignore_index).
 // Backward: one more pass writes
 //   dS = g_ce / N_ce (softmax(s) - onehot(y)) + g_kl T / N (softmax(s/T) - softmax(t/T)).
-// At T = 1 (the trainer's default) s/T is s: both passes then take one
-// exponential of s per logit instead of two (UNIT).
+// At T = 1 (the trainer's default) s/T is s, and at T = 2 e^s is the square of
+// e^(s/2): both passes then take one exponential of s per logit instead of two
+// (LossT).  The forward at other T is bound by its three exponentials and about
+// twenty more VALU operations per logit, not by memory.
 #include <cfloat>
+#include <type_traits>
 
 #include "vq_internal.h"
 
@@ -24,7 +27,18 @@ namespace vq {
 
 namespace {
 
-constexpr int kLossThreads = 256;
+// Threads per row: few rows leave CUs idle, so each takes a larger workgroup
+// there (MI355X, 64 x 151936, T = 2: forward 37 -> 30 us, backward 37 -> 26 us;
+// before, without the loads ahead, 55 and 52 us).  At 400 x 32000 a thread would
+// have four loads left to sum, and the larger workgroup's reduction loses:
+// forward 20 -> 22 us.
+constexpr int kLossThreads = 256, kLossFewThreads = 1024, kLossFewRows = 512, kLossFewVocab = 1 << 16;
+// Logits past this size do not stay in the last-level cache (256 MiB, shared by
+// both models' logits and the gradient) from one pass to the next: they are then
+// streamed past it.  2048 x 151936: forward 226 -> 199 us, backward 380 -> 357 us
+// (the loads of the next 8 logits ahead of the sums included); 1000 x 32000,
+// which fits, 32 -> 35 us for a streamed backward.
+constexpr int64_t kLossStreamBytes = (int64_t)128 << 20;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -35,15 +49,23 @@ constexpr float kLn2 = 0.6931471805599453f;
 // they would give are below 2^-126 times the loss weights.
 __device__ __forceinline__ float fexp(float x) { return __builtin_amdgcn_exp2f(x * kLog2e); }
 
-__device__ __forceinline__ void load8_bf16(const bf16_t* p, float (&v)[8]) {
-    const uint4 q = *reinterpret_cast<const uint4*>(p);
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+template <bool STREAM>
+__device__ __forceinline__ u32x4 load_logits(const bf16_t* p) {
+    const u32x4* q = reinterpret_cast<const u32x4*>(p);
+    return STREAM ? __builtin_nontemporal_load(q) : *q;
+}
+
+__device__ __forceinline__ void unpack8(const u32x4& w, float (&v)[8]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         v[2 * i] = __uint_as_float(w[i] << 16);
         v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
     }
 }
+
+// How the exponentials of s and of s / T go together: apart, as one (T = 1),
+// or e^s as the square of e^(s / 2) (T = 2).
+enum LossT : int { ANY_T = 0, UNIT_T = 1, TWO_T = 2 };
 
 // (m, z): z = sum exp(x - m).  Merge b into a.
 __device__ __forceinline__ void lse_merge(float& ma, float& za, float mb, float zb) {
@@ -82,51 +104,79 @@ __device__ __forceinline__ RowAcc shfl_acc(const RowAcc& a, int lane) {
 
 }  // namespace
 
-template <bool UNIT>
-__global__ __launch_bounds__(kLossThreads) void distill_fwd_kernel(const bf16_t* __restrict__ S,
+// Running sums over 8 more logits of each model.
+template <LossT LT>
+__device__ __forceinline__ void loss_accumulate(RowAcc& a, const float (&sv)[8], const float (&tv)[8], float inv_tau) {
+    float cs = sv[0], ct = tv[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) {
+        cs = fmaxf(cs, sv[j]);
+        ct = fmaxf(ct, tv[j]);
+    }
+    // rescale the running sums once per 8 values
+    const float nt = fmaxf(a.mt, LT == UNIT_T ? ct : ct * inv_tau);
+    const float ft = fexp(a.mt - nt);
+    a.zt *= ft;
+    a.at *= ft;
+    a.mt = nt;
+    if constexpr (LT != TWO_T) {
+        const float ns = fmaxf(a.ms, cs);
+        a.zs *= fexp(a.ms - ns);
+        a.ms = ns;
+    }
+    if constexpr (LT != UNIT_T) {
+        const float nq = fmaxf(a.mq, cs * inv_tau);
+        const float fq = fexp(a.mq - nq);
+        a.zq *= fq;
+        if constexpr (LT == TWO_T) a.zs *= fq * fq;
+        a.mq = nq;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if constexpr (LT != TWO_T) a.zs += fexp(sv[j] - a.ms);
+        if constexpr (LT != UNIT_T) {
+            const float eq = fexp(sv[j] * inv_tau - a.mq);
+            a.zq += eq;
+            if constexpr (LT == TWO_T) a.zs = fmaf(eq, eq, a.zs);
+        }
+        const float e = fexp((LT == UNIT_T ? tv[j] : tv[j] * inv_tau) - nt);
+        a.zt += e;
+        a.at += e > 0.f ? e * (tv[j] - sv[j]) : 0.f;
+    }
+}
+
+template <LossT LT, bool STREAM, int THREADS>
+__global__ __launch_bounds__(THREADS) void distill_fwd_kernel(const bf16_t* __restrict__ S,
                                                                    const bf16_t* __restrict__ Tl,
                                                                    const int64_t* __restrict__ labels, int64_t V,
                                                                    float inv_tau, float tau2,
                                                                    float* __restrict__ stats,
                                                                    float* __restrict__ row_loss) {
-    __shared__ RowAcc part[kLossThreads / 64];
+    __shared__ RowAcc part[THREADS / 64];
     const int64_t r = blockIdx.x;
     const bf16_t* s = S + r * V;
     const bf16_t* t = Tl + r * V;
     RowAcc a{-FLT_MAX, 0.f, -FLT_MAX, 0.f, -FLT_MAX, 0.f, 0.f};
-    for (int64_t i = (int64_t)threadIdx.x * 8; i < V; i += kLossThreads * 8) {
-        float sv[8], tv[8];
-        load8_bf16(s + i, sv);
-        load8_bf16(t + i, tv);
-        float cs = sv[0], ct = tv[0];
-#pragma unroll
-        for (int j = 1; j < 8; ++j) {
-            cs = fmaxf(cs, sv[j]);
-            ct = fmaxf(ct, tv[j]);
-        }
-        // rescale the running sums once per 8 values
-        const float ns = fmaxf(a.ms, cs), nt = fmaxf(a.mt, UNIT ? ct : ct * inv_tau);
-        a.zs *= fexp(a.ms - ns);
-        const float ft = fexp(a.mt - nt);
-        a.zt *= ft;
-        a.at *= ft;
-        a.ms = ns;
-        a.mt = nt;
-        if constexpr (!UNIT) {
-            const float nq = fmaxf(a.mq, cs * inv_tau);
-            a.zq *= fexp(a.mq - nq);
-            a.mq = nq;
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            a.zs += fexp(sv[j] - ns);
-            if constexpr (!UNIT) a.zq += fexp(sv[j] * inv_tau - a.mq);
-            const float e = fexp((UNIT ? tv[j] : tv[j] * inv_tau) - nt);
-            a.zt += e;
-            a.at += e > 0.f ? e * (tv[j] - sv[j]) : 0.f;
-        }
+    // the next 8 logits of each are in flight while these are summed
+    const int64_t step = THREADS * 8;
+    int64_t i = (int64_t)threadIdx.x * 8;
+    u32x4 qs, qt;
+    if (i < V) {
+        qs = load_logits<STREAM>(s + i);
+        qt = load_logits<STREAM>(t + i);
     }
-    if constexpr (UNIT) {
+    for (; i < V; i += step) {
+        float sv[8], tv[8];
+        unpack8(qs, sv);
+        unpack8(qt, tv);
+        if (i + step < V) {
+            qs = load_logits<STREAM>(s + i + step);
+            qt = load_logits<STREAM>(t + i + step);
+        }
+        loss_accumulate<LT>(a, sv, tv, inv_tau);
+    }
+    if constexpr (LT == TWO_T) a.ms = fmaxf(2.0f * a.mq, -FLT_MAX);  // a thread without logits: not -inf
+    if constexpr (LT == UNIT_T) {
         a.mq = a.ms;
         a.zq = a.zs;
     }
@@ -141,7 +191,7 @@ __global__ __launch_bounds__(kLossThreads) void distill_fwd_kernel(const bf16_t*
     if (threadIdx.x == 0) {
         RowAcc w = part[0];
 #pragma unroll
-        for (int k = 1; k < kLossThreads / 64; ++k) acc_merge(w, part[k]);
+        for (int k = 1; k < THREADS / 64; ++k) acc_merge(w, part[k]);
         const float lse_s = w.ms + __log2f(w.zs) * kLn2;
         const float lse_q = w.mq + __log2f(w.zq) * kLn2;
         const float lse_t = w.mt + __log2f(w.zt) * kLn2;
@@ -188,8 +238,8 @@ __global__ __launch_bounds__(256) void distill_reduce_kernel(const float* __rest
     }
 }
 
-template <bool UNIT>
-__global__ __launch_bounds__(kLossThreads) void distill_bwd_kernel(const bf16_t* __restrict__ S,
+template <LossT LT, bool STREAM, int THREADS>
+__global__ __launch_bounds__(THREADS) void distill_bwd_kernel(const bf16_t* __restrict__ S,
                                                                    const bf16_t* __restrict__ Tl,
                                                                    const int64_t* __restrict__ labels, int64_t V,
                                                                    float inv_tau, float tau,
@@ -205,25 +255,62 @@ __global__ __launch_bounds__(kLossThreads) void distill_bwd_kernel(const bf16_t*
     const int64_t y = labels[r];
     const float a = y != -100 ? grad_out[0] * aux[0] : 0.f;  // dL/dCE_mean / N_ce
     const float b = grad_out[1] * tau * aux[1];              // dL/dKL_mean * T^2 / T / N
-    for (int64_t i = (int64_t)threadIdx.x * 8; i < V; i += kLossThreads * 8) {
+    // T = 2: softmax(s) = softmax(s/2)^2 e^(2 lse_q - lse_s)
+    const float square = LT == TWO_T ? fexp(2.0f * lse_q - lse_s) : 0.f;
+    const int64_t step = THREADS * 8;
+    int64_t i = (int64_t)threadIdx.x * 8;
+    u32x4 qs, qt;
+    if (i < V) {
+        qs = load_logits<STREAM>(s + i);
+        qt = load_logits<STREAM>(t + i);
+    }
+    for (; i < V; i += step) {
         float sv[8], tv[8], g[8];
-        load8_bf16(s + i, sv);
-        load8_bf16(t + i, tv);
+        unpack8(qs, sv);
+        unpack8(qt, tv);
+        if (i + step < V) {
+            qs = load_logits<STREAM>(s + i + step);
+            qt = load_logits<STREAM>(t + i + step);
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float es = fexp(sv[j] - lse_s);
+            const float eq = LT == UNIT_T ? 0.f : fexp(sv[j] * inv_tau - lse_q);
+            const float es = LT == TWO_T ? eq * eq * square : fexp(sv[j] - lse_s);
             const float ps = es - ((i + j) == y ? 1.f : 0.f);
-            const float dq = UNIT ? es - fexp(tv[j] - lse_t)
-                                  : fexp(sv[j] * inv_tau - lse_q) - fexp(tv[j] * inv_tau - lse_t);
+            const float dq = LT == UNIT_T ? es - fexp(tv[j] - lse_t) : eq - fexp(tv[j] * inv_tau - lse_t);
             g[j] = a * ps + b * dq;
         }
-        uint4 q;
-        q.x = f2bf2(g[0], g[1]);
-        q.y = f2bf2(g[2], g[3]);
-        q.z = f2bf2(g[4], g[5]);
-        q.w = f2bf2(g[6], g[7]);
-        *reinterpret_cast<uint4*>(d + i) = q;
+        u32x4 q;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q[j] = f2bf2(g[2 * j], g[2 * j + 1]);
+        if constexpr (STREAM)
+            __builtin_nontemporal_store(q, reinterpret_cast<u32x4*>(d + i));
+        else
+            *reinterpret_cast<u32x4*>(d + i) = q;
     }
+}
+
+// The instantiation of a pass for these sizes and this temperature.
+template <class Launch>
+static void loss_dispatch(int64_t rows, int64_t V, float temperature, Launch launch) {
+    auto with_threads = [&](auto lt, auto stream) {
+        if (rows < kLossFewRows && V >= kLossFewVocab)
+            launch(lt, stream, std::integral_constant<int, kLossFewThreads>{});
+        else
+            launch(lt, stream, std::integral_constant<int, kLossThreads>{});
+    };
+    auto with_stream = [&](auto lt) {
+        if (2 * rows * V >= kLossStreamBytes)
+            with_threads(lt, std::true_type{});
+        else
+            with_threads(lt, std::false_type{});
+    };
+    if (temperature == 1.0f)
+        with_stream(std::integral_constant<LossT, UNIT_T>{});
+    else if (temperature == 2.0f)
+        with_stream(std::integral_constant<LossT, TWO_T>{});
+    else
+        with_stream(std::integral_constant<LossT, ANY_T>{});
 }
 
 hipError_t launch_distill_fwd(const bf16_t* S, const bf16_t* T, const int64_t* labels, int64_t rows, int64_t V,
@@ -231,12 +318,11 @@ hipError_t launch_distill_fwd(const bf16_t* S, const bf16_t* T, const int64_t* l
     float* stats = ws;
     float* row_loss = ws + 3 * rows;
     float* aux = ws + 5 * rows;
-    if (temperature == 1.0f)
-        distill_fwd_kernel<true><<<dim3((unsigned)rows), kLossThreads, 0, s>>>(S, T, labels, V, 1.0f, 1.0f, stats,
-                                                                            row_loss);
-    else
-        distill_fwd_kernel<false><<<dim3((unsigned)rows), kLossThreads, 0, s>>>(
-            S, T, labels, V, 1.0f / temperature, temperature * temperature, stats, row_loss);
+    loss_dispatch(rows, V, temperature, [&](auto lt, auto stream, auto threads) {
+        distill_fwd_kernel<decltype(lt)::value, decltype(stream)::value, decltype(threads)::value>
+            <<<dim3((unsigned)rows), decltype(threads)::value, 0, s>>>(S, T, labels, V, 1.0f / temperature,
+                                                                       temperature * temperature, stats, row_loss);
+    });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     distill_reduce_kernel<<<1, 256, 0, s>>>(row_loss, labels, rows, out, aux);
@@ -245,12 +331,11 @@ hipError_t launch_distill_fwd(const bf16_t* S, const bf16_t* T, const int64_t* l
 
 hipError_t launch_distill_bwd(const bf16_t* S, const bf16_t* T, const int64_t* labels, int64_t rows, int64_t V,
                               float temperature, const float* grad_out, bf16_t* dS, const float* ws, hipStream_t s) {
-    if (temperature == 1.0f)
-        distill_bwd_kernel<true><<<dim3((unsigned)rows), kLossThreads, 0, s>>>(S, T, labels, V, 1.0f, 1.0f, ws,
-                                                                            ws + 5 * rows, grad_out, dS);
-    else
-        distill_bwd_kernel<false><<<dim3((unsigned)rows), kLossThreads, 0, s>>>(
-            S, T, labels, V, 1.0f / temperature, temperature, ws, ws + 5 * rows, grad_out, dS);
+    loss_dispatch(rows, V, temperature, [&](auto lt, auto stream, auto threads) {
+        distill_bwd_kernel<decltype(lt)::value, decltype(stream)::value, decltype(threads)::value>
+            <<<dim3((unsigned)rows), decltype(threads)::value, 0, s>>>(S, T, labels, V, 1.0f / temperature, temperature,
+                                                                       ws, ws + 5 * rows, grad_out, dS);
+    });
     return hipGetLastError();
 }
 
