@@ -135,6 +135,15 @@ int vq_routed_linear_fwd(const uint16_t *x, int64_t m, int64_t n, int64_t d, int
                          const uint16_t *const *cand_bf16, const int32_t *perm, const int32_t *group_off,
                          uint16_t *y, void *stream);
 
+/* The token grouping vq_routed_linear_fwd takes, from one route per token
+ * (device int64 [m]): perm (device int32 [m]) lists the tokens of route 0,
+ * then of route 1, ..., each in token order; plan (device int32 [ncand + 2])
+ * holds group_off [ncand + 1], then the number of tokens whose route is
+ * outside [0, ncand) (they are in no group; perm ends in that many -1).
+ * Replaces the torch.argsort / bincount / cumsum a caller would write for
+ * voodoo_quant/layers.py:383-406. */
+int vq_route_tokens(const int64_t *routing, int64_t m, int ncand, int32_t *perm, int32_t *plan, void *stream);
+
 /* Embedding rows of the packed candidates (vocabulary [num_embeddings][d_pad],
  * every candidate's rows stored as d_pad/256 consecutive groups):
  *   routing == NULL: out[r][0:dim] = row ids[r] of

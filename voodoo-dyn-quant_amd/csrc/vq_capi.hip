@@ -371,6 +371,15 @@ int vq_routed_linear_fwd(const uint16_t* x, int64_t m, int64_t n, int64_t d, int
     return rc == VQ_OK ? ok() : rc;
 }
 
+int vq_route_tokens(const int64_t* routing, int64_t m, int ncand, int32_t* perm, int32_t* plan, void* stream) {
+    if (ncand < 1 || ncand > vq::kMaxCand) return fail(VQ_ERR_SHAPE, "ncand=%d out of [1, %d]", ncand, vq::kMaxCand);
+    if (m < 0 || m >= ((int64_t)1 << 31) - 1024) return fail(VQ_ERR_SHAPE, "m=%lld", (long long)m);
+    if (!plan || (m > 0 && (!routing || !perm))) return fail(VQ_ERR_NULL, "routing/perm/plan is NULL");
+    int rc = hip_check(vq::launch_route_tokens(routing, (int)m, ncand, perm, plan, static_cast<hipStream_t>(stream)),
+                       "route launch");
+    return rc == VQ_OK ? ok() : rc;
+}
+
 int vq_embedding_rows_fwd(int ncand, const int* qtypes, const void* const* qbytes, const float* probs,
                           const int64_t* routing, const int64_t* ids, int64_t nids, int64_t num_embeddings,
                           int64_t dim, int64_t d_pad, void* out, int out_f32, void* stream) {

@@ -425,7 +425,8 @@ struct StCfg {
     static int tiles_j(const GemmParams& p) { return (p.J + BJ - 1) / BJ; }
     static __host__ __device__ int ksteps(const GemmParams& p) { return (p.K + BK - 1) / BK; }
     // Fill in the work decomposition; returns the grid size (8 * items per XCD).
-    static int plan(GemmParams& p, int cus, bool split_ok) {
+    // per_round: kMinSavedPerRound applies (without it the plan bounds the workspace).
+    static int plan(GemmParams& p, int cus, bool split_ok, bool per_round = true) {
         if (p.I <= 0 || p.J <= 0) return 0;
         p.cus_per_xcd = cus / 8 > 0 ? cus / 8 : 1;
         p.tail_max = 0;
@@ -446,7 +447,8 @@ struct StCfg {
         // more for every whole round of tiles before it: behind many rounds a
         // half-empty last one costs less than its time, since the card is at
         // its power limit and the fewer CUs run it at a higher clock.
-        p.split_min_saved = EPI == EPI_STORE ? kMinSavedSplitSteps + kMinSavedPerRound * (tiles / (8 * p.cus_per_xcd)) : 0;
+        const int rounds = per_round ? tiles / (8 * p.cus_per_xcd) : 0;
+        p.split_min_saved = EPI == EPI_STORE ? kMinSavedSplitSteps + kMinSavedPerRound * rounds : 0;
         p.split_max = 8;
         p.split_ok = split_ok ? 1 : 0;
         for (int x = 0; x < 8; ++x) {

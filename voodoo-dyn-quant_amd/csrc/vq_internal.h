@@ -78,6 +78,8 @@ hipError_t launch_gate_dot(const CandGroup& cg, int N, int D, const float* dwp, 
 // PTQR: Y[perm[r]] = X[perm[r]] . W_g^T for r in [group_off[g], group_off[g+1])
 hipError_t launch_routed_fwd(const bf16_t* X, int M, int D, const bf16_t* const* cand_bf16, int64_t ldw, int N,
                              int ncand, const int* perm, const int* group_off, bf16_t* Y, hipStream_t s);
+// Stable grouping of m tokens by route (n candidates): perm [m], off [n + 2].
+hipError_t launch_route_tokens(const int64_t* routing, int m, int n, int* perm, int* off, hipStream_t s);
 hipError_t launch_gate_reduce(const float* partials, int64_t ntiles, int ncand, float* dprobs, hipStream_t s);
 // dprobs[k] = sum_t partials[t * stride + k], k < ncand
 hipError_t launch_gate_reduce_group(const float* partials, int64_t ntiles, int stride, const GateReduceOut& out,

@@ -31,6 +31,7 @@ _SIGNATURES = [
     ("vq_dequant_bf16", _i, [_i, _p, _p, _i64, _i64, _p]),
     ("vq_mix_weight", _i, [_i, _p, _p, _p, _i64, _i64, _p, _p]),
     ("vq_routed_linear_fwd", _i, [_p, _i64, _i64, _i64, _i64, _i, _p, _p, _p, _p, _p]),
+    ("vq_route_tokens", _i, [_p, _i64, _i, _p, _p, _p]),
     ("vq_embedding_rows_fwd", _i, [_i, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _i, _p]),
     ("vq_embedding_rows_bwd_workspace", _i64, [_i64, _i64, _i]),
     ("vq_embedding_rows_bwd", _i, [_i, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _i, _p, _p, _i64, _p]),
@@ -174,6 +175,19 @@ def routed_linear_fwd(x: torch.Tensor, cand_bf16, perm: torch.Tensor, group_off:
                                       _ptr_array(cand_bf16, "cand_bf16"), _dev_ptr(perm, "perm"),
                                       _dev_ptr(group_off, "group_off"), _dev_ptr(y, "y"), _stream(x.device)),
            "vq_routed_linear_fwd")
+
+
+def route_tokens(routing: torch.Tensor, ncand: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """(perm int32 [m], plan int32 [ncand + 2]) of one route per token (int64
+    [m]): perm groups the tokens by route in token order, plan[:ncand + 1] are
+    the group offsets and plan[ncand + 1] counts routes outside [0, ncand)."""
+    routing = _ids(routing, "routing")
+    perm = torch.empty(routing.numel(), dtype=torch.int32, device=routing.device)
+    plan = torch.empty(ncand + 2, dtype=torch.int32, device=routing.device)
+    _check(lib().vq_route_tokens(_dev_ptr(routing, "routing"), routing.numel(), ncand, _dev_ptr(perm, "perm"),
+                                 _dev_ptr(plan, "plan"), _stream(routing.device)),
+           "vq_route_tokens")
+    return perm, plan
 
 
 def _ids(t: torch.Tensor, name: str) -> torch.Tensor:

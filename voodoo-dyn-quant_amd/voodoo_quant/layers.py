@@ -609,12 +609,21 @@ class RoutedLinearFunction(Function):
         types, n, d_pad = meta
         x2 = _aligned(x)
         k = len(types)
-        r = routing.to(device=x2.device, dtype=torch.int64)
-        perm = torch.argsort(r, stable=True).to(torch.int32)
-        group_off = torch.zeros(k + 1, dtype=torch.int32, device=x2.device)
-        group_off[1:] = torch.cumsum(torch.bincount(r, minlength=k), 0).to(torch.int32)
+        r = routing.to(device=x2.device, dtype=torch.int64).contiguous()
+        if r.dim() != 1:
+            raise RuntimeError(f"routing must be one route per token, got shape {tuple(r.shape)}")
+        perm, plan = _hip.route_tokens(r, k)
+        # how many routes name no candidate, read behind an event while the
+        # product runs: the host waits for the grouping alone
+        stray = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        stray.copy_(plan[k + 1:], non_blocking=True)
+        grouped = torch.cuda.Event()
+        grouped.record(torch.cuda.current_stream(x2.device))
         y = torch.empty(x2.shape[0], n, dtype=torch.bfloat16, device=x2.device)
-        _hip.routed_linear_fwd(x2, cand_bf16, perm, group_off, n, d_pad, y)
+        _hip.routed_linear_fwd(x2, cand_bf16, perm, plan, n, d_pad, y)
+        grouped.synchronize()
+        if int(stray[0]):
+            raise RuntimeError(f"routing holds {int(stray[0])} routes outside [0, {k})")
         p = probs.detach().to(device=x2.device, dtype=torch.float32).contiguous()
         ctx.save_for_backward(x2, p)
         ctx.meta = meta
