@@ -155,7 +155,7 @@ int check_embed(int ncand, const int* qtypes, const void* const* qbytes, const i
     if (dim > d_pad) return fail(VQ_ERR_SHAPE, "embedding_dim=%lld exceeds d_pad=%lld", (long long)dim, (long long)d_pad);
     if (dim % 8 != 0) return fail(VQ_ERR_ALIGN, "embedding_dim=%lld must be a multiple of 8", (long long)dim);
     if (d_pad > (1 << 21)) return fail(VQ_ERR_SHAPE, "d_pad=%lld exceeds 2^21", (long long)d_pad);
-    if (vq::embed_plan(nids, dim).blocks >= ((int64_t)1 << 31))
+    if (nids * vq::embed_plan(nids, dim).nseg >= ((int64_t)1 << 31))
         return fail(VQ_ERR_SHAPE, "nids=%lld: too many rows for one launch", (long long)nids);
     if (nids > 0 && !ids) return fail(VQ_ERR_NULL, "ids is NULL");
     return VQ_OK;

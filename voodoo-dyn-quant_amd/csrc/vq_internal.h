@@ -8,12 +8,10 @@
 
 namespace vq {
 
-// Workgroup geometry of the streaming kernels: 256 threads, each decoding
-// kRunsPerThread runs of 8 weights, so one workgroup covers
-// kGroupsPerBlock groups of 256 weights.
+// Workgroup geometry of the streaming kernels: 256 threads of 16 weights, so
+// one pass of a workgroup covers kGroupsPerBlock groups of 256 weights.
 constexpr int kStreamThreads = 256;
-constexpr int kRunsPerThread = 2;
-constexpr int kGroupsPerBlock = kStreamThreads * 8 * kRunsPerThread / 256;  // 16
+constexpr int kGroupsPerBlock = kStreamThreads * 16 / 256;  // 16
 
 // Lets `kern` take `lds` bytes of dynamic LDS: above 64 KiB a kernel needs
 // the opt-in attribute (raised per kernel as larger sizes are asked for).
@@ -100,11 +98,12 @@ FusedPlan fused_plan(bool dx, int M, int N, int D);
 hipError_t launch_fused(bool dx, const bf16_t* act, const CandSet& cs, const float* probs, int M, int N, int D,
                         bf16_t* out, float* ws, hipStream_t s);
 
-// Embedding rows (vq_embed.hip): one workgroup per (requested row, segment of
-// at most kGroupsPerBlock groups); gused = groups covering dim.
+// Embedding rows (vq_embed.hip): a requested row is nseg segments of at most
+// seg <= kGroupsPerBlock groups, a workgroup takes `per` of them; gused =
+// groups covering dim.
 struct EmbedPlan {
-    int gused, nseg, seg;
-    int64_t blocks;  // nids * nseg; also the backward's partials per candidate
+    int gused, nseg, seg, per;
+    int64_t blocks;  // ceil(nids * nseg / per); also the backward's partials per candidate
 };
 EmbedPlan embed_plan(int64_t nids, int64_t dim);
 // out[r][0:dim] (bf16, or fp32 when out_f32) = row ids[r] of the mixture
