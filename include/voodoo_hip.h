@@ -75,7 +75,8 @@ int vq_mix_weight(int ncand, const int *qtypes, const void *const *qbytes, const
                   int64_t d_pad, uint16_t *w_eff, void *stream);
 
 /* Workspace bytes vq_gated_linear_fwd can use: fp32 partial tiles for the
- * K-split parts of the GEMM's last tiles (0 when the shape needs none). */
+ * K-split parts of the GEMM's last tiles, or partial sums for up to 8 tokens
+ * (0 when the shape needs none). */
 int64_t vq_gated_linear_fwd_workspace(int64_t m, int64_t n, int64_t d);
 
 /* y[m][n] = x[m][d] . w^T for a bf16 weight w[n][ldw] already in memory (the
@@ -89,8 +90,9 @@ int vq_linear_fwd(const uint16_t *x, int64_t m, int64_t n, int64_t d, const uint
 /* Forward of the gated Linear: mixes W_eff into `w_eff` ([n][d_pad] bf16,
  * caller-owned, kept for the backward) and writes y[m][n] = x[m][d] . W_eff^T.
  * `workspace` (optional, ws_bytes >= vq_gated_linear_fwd_workspace) lets the
- * GEMM split its last round of tiles along K; NULL runs them whole.  With
- * m == 0 it only mixes (x and y may then be NULL).
+ * GEMM split its last round of tiles along K, or a few tokens' products join
+ * the mixture's pass; NULL runs the mix and whole tiles.  With m == 0 it only
+ * mixes (x and y may then be NULL).
  * Replaces get_mixed_weight + F.linear in MixedQuantLinear.forward
  * (voodoo_quant/layers.py:1729-1731). */
 int vq_gated_linear_fwd(const uint16_t *x, int64_t m, int64_t n, int64_t d, int64_t d_pad, int ncand,
@@ -99,15 +101,17 @@ int vq_gated_linear_fwd(const uint16_t *x, int64_t m, int64_t n, int64_t d, int6
 
 /* Workspace bytes of vq_gated_linear_fwd_fused (dx == 0) or
  * vq_gated_linear_dx_fused (dx != 0): fp32 parts of the reduction, split
- * across workgroups when the output alone gives too few (0: no split). */
+ * across workgroups when the output alone gives too few, or sums of 256
+ * weights for up to 8 tokens (0: no split). */
 int64_t vq_gated_linear_fused_workspace(int64_t m, int64_t n, int64_t d, int dx);
 
 /* The gated Linear's products for few tokens with W_eff never in memory: each
  * workgroup decodes the K candidates' packed bytes for its 32-row x 256-weight
  * tiles into LDS, mixes them with probs in fp32 (fma(p_k dl, u, acc): within
  * a bf16 ulp of vq_mix_weight's W_eff, not bit-identical) and multiplies them
- * there.  The tiles are decoded again for every 32 tokens, so the caller
- * picks these below a measured token count and the materialising entry
+ * there.  For up to 8 tokens the forward multiplies the mixed fp32 weights as
+ * they are decoded, without tiles, and rounds only y.  The tiles are decoded
+ * again for every 32 tokens, so the caller picks these below a measured token count and the materialising entry
  * points above it.
  *   vq_gated_linear_fwd_fused: y[m][n] = x[m][d] . W_eff^T
  *     (replaces get_mixed_weight + F.linear, voodoo_quant/layers.py:1729-1731);

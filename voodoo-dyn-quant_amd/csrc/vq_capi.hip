@@ -693,7 +693,8 @@ int vq_distill_loss_bwd(const uint16_t* logits, const uint16_t* teacher_logits, 
 
 int64_t vq_gated_linear_fwd_workspace(int64_t m, int64_t n, int64_t d) {
     if (m < 0 || n <= 0 || d <= 0 || m > INT32_MAX || n > INT32_MAX || d > INT32_MAX) return -1;
-    return align256(vq::fwd_tail_bytes((int)m, (int)n, (int)d));
+    const int64_t tail = vq::fwd_tail_bytes((int)m, (int)n, (int)d), few = vq::few_fwd_bytes(m, n, d);
+    return align256(tail > few ? tail : few);
 }
 
 int vq_gated_linear_fwd(const uint16_t* x, int64_t m, int64_t n, int64_t d, int64_t d_pad, int ncand,
@@ -708,6 +709,13 @@ int vq_gated_linear_fwd(const uint16_t* x, int64_t m, int64_t n, int64_t d, int6
         return fail(VQ_ERR_ALIGN, "x/w_eff/y not 16-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const vq::CandSet cs = make_set(ncand, qtypes, qbytes, d_pad);
+    if (vq::few_fwd(cs, true, m, n, d) && workspace && aligned16(workspace) &&
+        ws_bytes >= vq::few_fwd_bytes(m, n, d)) {
+        rc = hip_check(vq::launch_few_fwd(x, cs, probs, (int)m, (int)n, (int)d, w_eff, y,
+                                          static_cast<float*>(workspace), s),
+                       "few-token forward launch");
+        return rc == VQ_OK ? ok() : rc;
+    }
     rc = hip_check(vq::launch_mix(cs, probs, w_eff, n * d_pad / 256, s), "mix launch");
     if (rc != VQ_OK) return rc;
     if (m == 0) return ok();
@@ -795,7 +803,9 @@ int vq_gated_linear_bwd_static(const uint16_t* dy, const uint16_t* x, int64_t m,
 int64_t vq_gated_linear_fused_workspace(int64_t m, int64_t n, int64_t d, int dx) {
     if (m < 0 || n <= 0 || d <= 0 || m > INT32_MAX || n > (1 << 21) || d > (1 << 21)) return -1;
     if (m == 0) return 0;
-    return align256(vq::fused_plan(dx != 0, (int)m, (int)n, (int)d).ws_bytes);
+    const int64_t tiles = vq::fused_plan(dx != 0, (int)m, (int)n, (int)d).ws_bytes;
+    const int64_t few = dx ? 0 : vq::few_fwd_bytes(m, n, d);
+    return align256(tiles > few ? tiles : few);
 }
 
 namespace {
@@ -813,8 +823,16 @@ int run_fused(bool dx, const uint16_t* act, int64_t m, int64_t n, int64_t d, int
         return fail(VQ_ERR_WORKSPACE, "workspace of %lld bytes required, got %lld", (long long)need,
                     (long long)(workspace ? ws_bytes : 0));
     if (workspace && !aligned16(workspace)) return fail(VQ_ERR_ALIGN, "workspace not 16-byte aligned");
-    rc = hip_check(vq::launch_fused(dx, act, make_set(ncand, qtypes, qbytes, d_pad), probs, (int)m, (int)n, (int)d,
-                                    out, need > 0 ? static_cast<float*>(workspace) : nullptr,
+    const vq::CandSet cs = make_set(ncand, qtypes, qbytes, d_pad);
+    if (!dx && vq::few_fwd(cs, false, m, n, d) && workspace && ws_bytes >= vq::few_fwd_bytes(m, n, d)) {
+        rc = hip_check(vq::launch_few_fwd(act, cs, probs, (int)m, (int)n, (int)d, nullptr, out,
+                                          static_cast<float*>(workspace),
+                                          static_cast<hipStream_t>(stream)),
+                       "few-token forward launch");
+        return rc == VQ_OK ? ok() : rc;
+    }
+    rc = hip_check(vq::launch_fused(dx, act, cs, probs, (int)m, (int)n, (int)d, out,
+                                    need > 0 ? static_cast<float*>(workspace) : nullptr,
                                     static_cast<hipStream_t>(stream)),
                    dx ? "fused dX launch" : "fused forward launch");
     return rc == VQ_OK ? ok() : rc;

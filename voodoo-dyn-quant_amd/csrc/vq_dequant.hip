@@ -368,6 +368,265 @@ hipError_t launch_mix(const CandSet& cs, const float* probs, bf16_t* w_eff, int6
 }
 
 // ---------------------------------------------------------------------------
+// The forward of up to kFewTokens tokens in the mixture's own pass: a
+// workgroup stages 16 consecutive groups of every candidate as the mix does,
+// and a thread's 16 mixed weights meet the tokens' activations in registers, so
+// no GEMM reads W_eff back.  WRITE: the mix kernel's W_eff, bit for bit, goes
+// to memory (a backward will read it) and the products take its bf16 values.
+// !WRITE: acc = fma(p_k dl, u, acc), c += p_k c_k, one operation per weight and
+// candidate where the separately rounded mixture takes three, and the
+// products take the fp32 weights unrounded; nothing but the group sums is
+// written.  The 16 threads of a group add up their products (DPP), and
+// few_reduce_kernel adds each output's ceil(D / 256) group sums in order, so
+// results do not depend on the launch.
+//
+// Bound: the packed bytes (346 MB at 17408 x 5120, K = 6, 58 us at 6 TB/s) and
+// the decode's VALU work (about as long) run side by side, from workgroups
+// that wait on their copies and others that decode.  Measured there on MI355X
+// at 1 token: 87 us, against 110 for the mix and 55 for the GEMM.
+// ---------------------------------------------------------------------------
+struct FewPlan {
+    CandSet cs;
+    const float* probs;
+    const bf16_t* x;   // [M][D]
+    bf16_t* w_eff;     // WRITE
+    float* part;       // [M][N][G] group sums
+    int64_t ngroups;
+    int M, N, D, G;    // G = ceil(D / 256): groups past D hold no column of x
+    int gbytes[kMaxCand];
+    int lds_off[kMaxCand];
+};
+
+// The sum of v over the 16 lanes of a DPP row, in every lane.
+__device__ __forceinline__ float row16_sum(float v) {
+    v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x128, 0xf, 0xf, true));
+    v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x124, 0xf, 0xf, true));
+    v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x122, 0xf, 0xf, true));
+    v += __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0x121, 0xf, 0xf, true));
+    return v;
+}
+
+__device__ __forceinline__ float dot16_bf16(const float (&w)[16], const u32x4& a, const u32x4& b) {
+    const uint32_t q[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        s0 = fmaf(w[2 * i], __uint_as_float(q[i] << 16), s0);
+        s1 = fmaf(w[2 * i + 1], __uint_as_float(q[i] & 0xffff0000u), s1);
+    }
+    return s0 + s1;
+}
+
+// MT: tokens, at most (the activations of the first min(MT, 4) are loaded ahead
+// of the wait for the candidates).  IQ as in mix_kernel.
+template <bool IQ, bool WRITE, int MT>
+__global__ __launch_bounds__(kStreamThreads, IQ || MT > 1 ? 4 : 8) void few_fwd_kernel(FewPlan fp) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int AHEAD = MT < 4 ? MT : 4;
+    const CandSet& cs = fp.cs;
+    const uint32_t g0 = blockIdx.x * (uint32_t)kMixGroupsPerPass;  // ngroups < 2^31
+    const int ng = min(kMixGroupsPerPass, (int)(fp.ngroups - g0));
+    const int t = threadIdx.x, j = t >> 4, p = kMixRun * (t & 15);
+    // group g0 + j: weight row n, columns 256 grp + p ..
+    const uint32_t rg = (uint32_t)cs.row_groups;
+    const uint32_t row0 = g0 / rg;
+    const uint32_t at = g0 - row0 * rg + (uint32_t)j;
+    const int n = (int)(row0 + at / rg), grp = (int)(at % rg);
+    const int col = 256 * grp + p;
+    const bool lo = j < ng && col < fp.D, hi = j < ng && col + 8 < fp.D;  // D is a multiple of 8
+    // Activations and probabilities are asked for before the copies, so they
+    // never wait behind them.  A load past the M rows, or masked off, returns
+    // zeros by its bounds check, with no branch around it.
+    const __amdgpu_buffer_rsrc_t xr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(fp.x), (short)0, fp.M * fp.D * 2, 0x00020000);
+    const int out_of_range = INT32_MIN;  // unsigned 2^31: past the 2^25 bytes of x at most
+    auto load_x = [&](int m, u32x4& a, u32x4& b) {
+        const int off = 2 * (m * fp.D + col);
+        a = __builtin_amdgcn_raw_buffer_load_b128(xr, lo ? off : out_of_range, 0, 0);
+        b = __builtin_amdgcn_raw_buffer_load_b128(xr, hi ? off + 16 : out_of_range, 0, 0);
+    };
+    u32x4 xa[AHEAD], xb[AHEAD];
+#pragma unroll
+    for (int m = 0; m < AHEAD; ++m) load_x(m, xa[m], xb[m]);
+    const float probs = fp.probs[min(t & 63, cs.ncand - 1)];  // candidate k's in lane k
+    for (int k = 0; k < cs.ncand; ++k) {
+        const int gb = fp.gbytes[k];
+        stage_bytes(lds + fp.lds_off[k], cs.qbytes[k] + (int64_t)g0 * gb, ng * gb);
+    }
+    stage_wait();
+    __syncthreads();
+    // groups past the last one decode stale LDS (every code-book index stays
+    // inside its book) and store nothing, so every lane of a readlane is live
+    float w[kMixRun];
+#pragma unroll
+    for (int r = 0; r < kMixRun; ++r) w[r] = 0.0f;
+    float off = 0.0f;
+    for (int k = 0; k < cs.ncand; ++k) {
+        const int qt = cs.qtype[k];
+        const uint8_t* g = lds + fp.lds_off[k] + j * fp.gbytes[k];
+        const float pk = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(probs), k));
+        uint32_t uw[kMixRun / 4];
+        float dl, c;
+        switch (qt) {
+        case Q8_0: decode_affine<Q8_0, kMixRun>(g, p, uw, dl, c); break;
+        case Q2_K: decode_affine<Q2_K, kMixRun>(g, p, uw, dl, c); break;
+        case Q3_K: decode_affine<Q3_K, kMixRun>(g, p, uw, dl, c); break;
+        case Q4_K: decode_affine<Q4_K, kMixRun>(g, p, uw, dl, c); break;
+        case Q5_K: decode_affine<Q5_K, kMixRun>(g, p, uw, dl, c); break;
+        case Q6_K: decode_affine<Q6_K, kMixRun>(g, p, uw, dl, c); break;
+        default:
+            if constexpr (IQ)
+                decode_affine_iq<kMixRun>(qt, g, p, uw, dl, c);
+            else
+                decode_affine<Q6_K, kMixRun>(g, p, uw, dl, c);
+            break;
+        }
+        opaque_words(uw);
+        if constexpr (WRITE) {
+            // mix_kernel's arithmetic: each weight rounded once, then product
+            // and sum rounded separately
+#pragma unroll
+            for (int r = 0; r < kMixRun; ++r) {
+#pragma clang fp contract(off)
+                const float wk = fmaf(dl, (float)((uw[r >> 2] >> (8 * (r & 3))) & 0xffu), c);
+                w[r] = w[r] + pk * wk;
+            }
+        } else {
+            const float pdl = pk * dl;
+            off = fmaf(pk, c, off);
+#pragma unroll
+            for (int r = 0; r < kMixRun; ++r)
+                w[r] = fmaf(pdl, (float)((uw[r >> 2] >> (8 * (r & 3))) & 0xffu), w[r]);
+        }
+    }
+    if constexpr (WRITE) {
+        uint32_t v[kMixRun / 2];
+#pragma unroll
+        for (int i = 0; i < kMixRun / 2; ++i) {
+            v[i] = f2bf2(w[2 * i], w[2 * i + 1]);
+            w[2 * i] = __uint_as_float(v[i] << 16);
+            w[2 * i + 1] = __uint_as_float(v[i] & 0xffff0000u);
+        }
+        if (j < ng) {
+            uint4* o = reinterpret_cast<uint4*>(fp.w_eff + ((int64_t)g0 + j) * 256 + p);
+            o[0] = make_uint4(v[0], v[1], v[2], v[3]);
+            o[1] = make_uint4(v[4], v[5], v[6], v[7]);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kMixRun; ++r) w[r] += off;
+    }
+    // columns past D meet no activation, whatever their weights hold
+#pragma unroll
+    for (int r = 0; r < kMixRun; ++r) w[r] = (r < 8 ? lo : hi) ? w[r] : 0.0f;
+    float mine = 0.0f;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        if (m >= fp.M) break;
+        u32x4 a, b;
+        if (m < AHEAD) {
+            a = xa[m < AHEAD ? m : 0];
+            b = xb[m < AHEAD ? m : 0];
+        } else {
+            load_x(m, a, b);
+        }
+        const float s = row16_sum(dot16_bf16(w, a, b));
+        if ((t & 15) == m) mine = s;
+    }
+    if (j < ng && (t & 15) < fp.M && grp < fp.G)
+        fp.part[((int64_t)(t & 15) * fp.N + n) * fp.G + grp] = mine;
+}
+
+// y[i] = bf16(sum of part[i * G .. i * G + G)), i = m N + n: 16 lanes per output.
+__global__ __launch_bounds__(kStreamThreads) void few_reduce_kernel(const float* __restrict__ part, int64_t count,
+                                                                    int G, bf16_t* __restrict__ y) {
+    const int lane = threadIdx.x & 15;
+    const int64_t i = (int64_t)blockIdx.x * (kStreamThreads / 16) + (threadIdx.x >> 4);
+    if (i >= count) return;  // whole DPP rows
+    float s = 0.0f;
+    for (int g = lane; g < G; g += 16) s += part[i * G + g];
+    s = row16_sum(s);
+    if (lane == 0) y[i] = f2bf(s);
+}
+
+int64_t few_fwd_bytes(int64_t M, int64_t N, int64_t D) {
+    return M >= 1 && M <= kFewTokens ? M * N * ((D + 255) / 256) * (int64_t)sizeof(float) : 0;
+}
+
+// A token costs this pass about 45 instructions per 16 weights, the general
+// path nearly nothing until its tiles fill, so each kind of pass has a token
+// count from which mix + GEMM is the faster one.  Measured on MI355X, this pass
+// against the faster of the mix + GEMM and the tile-fused path, us:
+//   up to 2^22 weights launches count: 2048 x 2048, K = 6, W_eff kept, 1 / 8
+//   tokens 12.4 / 14.3 against 28, not kept 9.8 / 11.6 against 18; K = 8 with
+//   code books, 8 tokens, 17.9 against 31 and 14.4 against 23;
+//   17408 x 5120, K = 6 (164-167): not kept 87 / 97 / 114 / 145 at 1 / 2 / 4 / 8
+//   tokens, kept 133 / 140 / 154 / 188; K = 8 with code books (229; more
+//   registers, fewer waves): not kept 162 / 164 / 204 / 231, kept 199 / 200 /
+//   234 / 262.  5120 x 17408 and 6144 x 5120 cross at the same counts.
+bool few_fwd(const CandSet& cs, bool keep_w_eff, int64_t M, int64_t N, int64_t D) {
+    if (M < 1 || M > kFewTokens || N * cs.row_groups >= ((int64_t)1 << 31)) return false;
+    if (N * D <= ((int64_t)1 << 22)) return true;
+    const int half = any_iq(cs) ? 2 : 1;
+    return M <= (keep_w_eff ? 4 : kFewTokens) / half;
+}
+
+template <bool IQ, bool WRITE>
+static hipError_t launch_few_t(const FewPlan& fp, dim3 grid, size_t lds, hipStream_t s) {
+    const void* kern = fp.M == 1   ? (const void*)few_fwd_kernel<IQ, WRITE, 1>
+                       : fp.M == 2 ? (const void*)few_fwd_kernel<IQ, WRITE, 2>
+                       : fp.M <= 4 ? (const void*)few_fwd_kernel<IQ, WRITE, 4>
+                                   : (const void*)few_fwd_kernel<IQ, WRITE, kFewTokens>;
+    const hipError_t e = allow_dynamic_lds(kern, lds);  // 16 Q8_0 candidates stage 68 KiB
+    if (e != hipSuccess) return e;
+    if (fp.M == 1)
+        few_fwd_kernel<IQ, WRITE, 1><<<grid, kStreamThreads, lds, s>>>(fp);
+    else if (fp.M == 2)
+        few_fwd_kernel<IQ, WRITE, 2><<<grid, kStreamThreads, lds, s>>>(fp);
+    else if (fp.M <= 4)
+        few_fwd_kernel<IQ, WRITE, 4><<<grid, kStreamThreads, lds, s>>>(fp);
+    else
+        few_fwd_kernel<IQ, WRITE, kFewTokens><<<grid, kStreamThreads, lds, s>>>(fp);
+    return hipGetLastError();
+}
+
+hipError_t launch_few_fwd(const bf16_t* x, const CandSet& cs, const float* probs, int M, int N, int D, bf16_t* w_eff,
+                          bf16_t* y, float* part, hipStream_t s) {
+    if (M < 1 || M > kFewTokens || D % 8 != 0 || !part || (int64_t)(D + 255) / 256 > cs.row_groups ||
+        (int64_t)N * cs.row_groups >= ((int64_t)1 << 31))
+        return hipErrorInvalidValue;
+    FewPlan fp{};
+    fp.cs = cs;
+    fp.probs = probs;
+    fp.x = x;
+    fp.w_eff = w_eff;
+    fp.part = part;
+    fp.ngroups = (int64_t)N * cs.row_groups;
+    fp.M = M;
+    fp.N = N;
+    fp.D = D;
+    fp.G = (D + 255) / 256;
+    size_t lds = 0;
+    for (int k = 0; k < cs.ncand; ++k) {
+        fp.gbytes[k] = group_bytes(cs.qtype[k]);
+        fp.lds_off[k] = (int)lds;
+        lds += (kMixGroupsPerPass * fp.gbytes[k] + 15) & ~15;
+    }
+    const dim3 grid((unsigned)((fp.ngroups + kMixGroupsPerPass - 1) / kMixGroupsPerPass));
+    const bool iq = any_iq(cs);
+    hipError_t e;
+    if (w_eff)
+        e = iq ? launch_few_t<true, true>(fp, grid, lds, s) : launch_few_t<false, true>(fp, grid, lds, s);
+    else
+        e = iq ? launch_few_t<true, false>(fp, grid, lds, s) : launch_few_t<false, false>(fp, grid, lds, s);
+    if (e != hipSuccess) return e;
+    const int64_t count = (int64_t)M * N;
+    few_reduce_kernel<<<dim3((unsigned)((count + kStreamThreads / 16 - 1) / (kStreamThreads / 16))), kStreamThreads, 0,
+                        s>>>(part, count, fp.G, y);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Gate dots from dW parts (the EPI_PARTS gate product):
 //   partials[block][set * kstride + k] = sum over the block's weights of
 //   dW[n][d] * W_k[n][d],

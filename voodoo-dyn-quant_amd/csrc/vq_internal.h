@@ -24,6 +24,17 @@ hipError_t launch_mix(const CandSet& cs, const float* probs, bf16_t* w_eff, int6
 hipError_t launch_mix_sets(int nsets, const CandSet* sets, const float* const* probs, bf16_t* const* out,
                            const int64_t* ngroups, hipStream_t s);
 
+// Forward of at most kFewTokens tokens in the mixture's pass (vq_dequant.hip):
+// Y[M][N] = X[M][D] . W_eff^T without reading W_eff back.  w_eff: written as
+// launch_mix writes it, or NULL (the products then take the unrounded fp32
+// mixture).  few_fwd: whether this pass is the faster one.  part:
+// few_fwd_bytes(M, N, D) of fp32 workspace (0: M out of range).
+constexpr int kFewTokens = 8;
+bool few_fwd(const CandSet& cs, bool keep_w_eff, int64_t M, int64_t N, int64_t D);
+int64_t few_fwd_bytes(int64_t M, int64_t N, int64_t D);
+hipError_t launch_few_fwd(const bf16_t* x, const CandSet& cs, const float* probs, int M, int N, int D, bf16_t* w_eff,
+                          bf16_t* y, float* part, hipStream_t s);
+
 // Gated-Linear GEMMs (vq_gemm.hip).  All matrices are row-major bf16.
 //   fwd:  Y[M][N]  = X[M][D] . W[N][D]^T          (W row stride ldw)
 //   dx:   dX[M][D] = dY[M][N] . W[N][D]

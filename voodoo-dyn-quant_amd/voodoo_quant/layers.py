@@ -254,6 +254,22 @@ def use_fused(m: int, n: int, d_pad: int) -> bool:
     return FUSED_PRODUCTS and 0 < m <= FUSED_MAX_TOKENS and n <= FUSED_MAX_ROWS and n * d_pad <= FUSED_MAX_WEIGHTS
 
 
+# A forward without a backward: at these token counts vq_gated_linear_fwd_fused
+# multiplies in the mixture's own pass whatever the tensor's size, and W_eff is
+# neither written nor read.  Measured on MI355X, 17408 x 5120, against mix +
+# GEMM: K-quants (K = 6) 87 us at 1 token and 145 at 8, against 167; with
+# code-book formats (K = 8) 162 at 1 token and 204 at 4, against 230, and
+# level at 8.
+FEW_TOKENS = 8
+FEW_TOKENS_IQ = 4
+_K_QUANT_IDS = frozenset((8, 10, 11, 12, 13, 14))
+
+
+def use_few(m: int, types) -> bool:
+    limit = FEW_TOKENS if _K_QUANT_IDS.issuperset(types) else FEW_TOKENS_IQ
+    return FUSED_PRODUCTS and 0 < m <= limit
+
+
 def _finish_on_gate_stream(stream, rows, grads, keep) -> None:
     """The gate gradients `grads`, reduced on `stream` by the library, are
     added to the sink rows there; every buffer that stream still reads or
@@ -286,7 +302,9 @@ class GatedLinearFunction(Function):
         m, d = x2.shape
         p = probs.detach().to(device=x.device, dtype=torch.float32).contiguous()
         y = torch.empty(m, n, dtype=torch.bfloat16, device=x.device)
-        ctx.fused = premixed is None and use_fused(m, n, d_pad)
+        # without a gradient nothing reads W_eff after this call
+        alone = sink is None and not any(ctx.needs_input_grad) and use_few(m, types)
+        ctx.fused = premixed is None and (alone or use_fused(m, n, d_pad))
         if premixed is not None:  # W_eff mixed ahead on the prefetch stream: the GEMM only
             nbytes = _hip.fwd_workspace_bytes(m, n, d)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes > 0 else None
