@@ -168,6 +168,12 @@ int vq_embedding_rows_fwd(int ncand, const int *qtypes, const void *const *qbyte
                           const int64_t *routing, const int64_t *ids, int64_t nids, int64_t num_embeddings,
                           int64_t dim, int64_t d_pad, void *out, int out_f32, void *stream);
 
+/* *out_of_range (device, 0 or 1) = whether any of the nids ids (device int64)
+ * lies outside [0, num_embeddings): the range check of a lookup whose host
+ * side reads the answer later.  One workgroup: meant for up to 2^16 ids. */
+int vq_ids_out_of_range(const int64_t *ids, int64_t nids, int64_t num_embeddings, uint8_t *out_of_range,
+                        void *stream);
+
 /* Workspace bytes vq_embedding_rows_bwd needs (one fp32 partial per
  * workgroup and candidate). */
 int64_t vq_embedding_rows_bwd_workspace(int64_t nids, int64_t dim, int ncand);

@@ -66,3 +66,13 @@ def test_rows_sharing_a_workgroup(dim, vocab, nids, types):
         for k, t in enumerate(terms):
             size = cands[k].abs().max().double() * dy.double().abs()[~bad].sum()
             assert (dp[k] - t.sum()).abs() <= 32 * 2.0**-24 * 4 * size + 2.0**-24 * t.sum().abs()
+
+
+@pytest.mark.parametrize("n,at,value", [(1, 0, 10), (1, 0, 9), (8192, 8191, -1), (8193, 8192, 10), (20000, 9000, 1 << 40),
+                                        (20000, 0, 0)])
+def test_id_range_check(n, at, value):
+    from voodoo_quant import _hip
+
+    ids = torch.arange(n) % 10
+    ids[at] = value
+    assert bool(_hip.ids_out_of_range(ids.cuda(), 10)[0]) == (not 0 <= value < 10)

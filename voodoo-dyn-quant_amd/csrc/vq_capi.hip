@@ -396,6 +396,17 @@ int vq_embedding_rows_fwd(int ncand, const int* qtypes, const void* const* qbyte
     return rc == VQ_OK ? ok() : rc;
 }
 
+int vq_ids_out_of_range(const int64_t* ids, int64_t nids, int64_t num_embeddings, uint8_t* out_of_range,
+                        void* stream) {
+    if (nids < 0 || nids > INT32_MAX || num_embeddings <= 0)
+        return fail(VQ_ERR_SHAPE, "nids=%lld num_embeddings=%lld", (long long)nids, (long long)num_embeddings);
+    if ((nids > 0 && !ids) || !out_of_range) return fail(VQ_ERR_NULL, "ids/out_of_range is NULL");
+    const int rc = hip_check(vq::launch_ids_out_of_range(ids, (int)nids, num_embeddings, out_of_range,
+                                                         static_cast<hipStream_t>(stream)),
+                             "id check launch");
+    return rc == VQ_OK ? ok() : rc;
+}
+
 int64_t vq_embedding_rows_bwd_workspace(int64_t nids, int64_t dim, int ncand) {
     if (nids < 0 || dim <= 0 || ncand < 1 || ncand > vq::kMaxCand) return -1;
     return align256(vq::embed_plan(nids, dim).blocks * ncand * (int64_t)sizeof(float));

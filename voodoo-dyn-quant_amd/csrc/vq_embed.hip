@@ -298,6 +298,31 @@ __global__ __launch_bounds__(kStreamThreads) void embed_rows_bwd_kernel(CandSet 
     }
 }
 
+// One workgroup, so that the answer needs no cleared flag and no second launch;
+// a thread keeps 8 ids in flight.  Launches bound the check it serves: as torch
+// comparisons and an any() it took five.
+__global__ __launch_bounds__(1024) void ids_out_of_range_kernel(const int64_t* __restrict__ ids, int nids,
+                                                                int64_t vocab, uint8_t* __restrict__ bad) {
+    bool mine = false;
+    for (int64_t i0 = threadIdx.x; i0 < nids; i0 += 8 * 1024) {
+        int64_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int64_t i = i0 + 1024 * u;
+            v[u] = ids[i < nids ? i : nids - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) mine = mine || v[u] < 0 || v[u] >= vocab;
+    }
+    const int any = __syncthreads_or(mine);
+    if (threadIdx.x == 0) *bad = any ? 1 : 0;
+}
+
+hipError_t launch_ids_out_of_range(const int64_t* ids, int nids, int64_t vocab, uint8_t* bad, hipStream_t s) {
+    ids_out_of_range_kernel<<<1, 1024, 0, s>>>(ids, nids, vocab, bad);
+    return hipGetLastError();
+}
+
 EmbedPlan embed_plan(int64_t nids, int64_t dim) {
     EmbedPlan pl;
     pl.gused = (int)((dim + 255) / 256);

@@ -121,6 +121,8 @@ EmbedPlan embed_plan(int64_t nids, int64_t dim);
 // (routing NULL) or of candidate routing[r]
 hipError_t launch_embed_rows(const CandSet& cs, const float* probs, const int64_t* routing, const int64_t* ids,
                              int64_t nids, int64_t vocab, int64_t dim, void* out, bool out_f32, hipStream_t s);
+// *bad = whether any of ids[0 .. nids) lies outside [0, vocab)
+hipError_t launch_ids_out_of_range(const int64_t* ids, int nids, int64_t vocab, uint8_t* bad, hipStream_t s);
 // dprobs[k] = sum_r <grad[r][0:dim], W_k[ids[r]][0:dim]> (grad bf16, or fp32
 // when grad_f32); partials: embed_plan(...).blocks * ncand floats
 hipError_t launch_embed_rows_bwd(const CandSet& cs, const int64_t* ids, int64_t nids, int64_t vocab, int64_t dim,

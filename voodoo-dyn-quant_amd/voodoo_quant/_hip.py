@@ -32,6 +32,7 @@ _SIGNATURES = [
     ("vq_mix_weight", _i, [_i, _p, _p, _p, _i64, _i64, _p, _p]),
     ("vq_routed_linear_fwd", _i, [_p, _i64, _i64, _i64, _i64, _i, _p, _p, _p, _p, _p]),
     ("vq_route_tokens", _i, [_p, _i64, _i, _p, _p, _p]),
+    ("vq_ids_out_of_range", _i, [_p, _i64, _i64, _p, _p]),
     ("vq_embedding_rows_fwd", _i, [_i, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _i, _p]),
     ("vq_embedding_rows_bwd_workspace", _i64, [_i64, _i64, _i]),
     ("vq_embedding_rows_bwd", _i, [_i, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _i, _p, _p, _i64, _p]),
@@ -194,6 +195,16 @@ def _ids(t: torch.Tensor, name: str) -> torch.Tensor:
     if t.dtype != torch.int64:
         raise ValueError(f"{name} must be int64, got {t.dtype}")
     return t
+
+
+def ids_out_of_range(ids: torch.Tensor, num_embeddings: int) -> torch.Tensor:
+    """bool [1] on ids' device: whether any id (int64) lies outside [0, num_embeddings)."""
+    ids = _ids(ids, "ids")
+    bad = torch.empty(1, dtype=torch.bool, device=ids.device)
+    _check(lib().vq_ids_out_of_range(_dev_ptr(ids, "ids"), ids.numel(), num_embeddings,
+                                     _dev_ptr(bad, "out_of_range"), _stream(ids.device)),
+           "vq_ids_out_of_range")
+    return bad
 
 
 def embedding_rows_fwd(ggml_types, qbytes, probs: torch.Tensor | None, routing: torch.Tensor | None,

@@ -120,6 +120,9 @@ def _sample_token_routing(probs: torch.Tensor, num_tokens: int) -> torch.Tensor:
 # host flag, event after its copy).
 _PENDING_ID_CHECKS: list = []
 _MAX_PENDING_ID_CHECKS = 64
+# Up to here one workgroup's launch checks the ids (it takes 8192 a pass);
+# above, torch's launches over the whole chip.
+_ONE_BLOCK_IDS = 1 << 16
 
 
 def check_embedding_ids(ids: torch.Tensor, num_embeddings: int, name: str, mode: str) -> None:
@@ -146,7 +149,10 @@ def check_embedding_ids(ids: torch.Tensor, num_embeddings: int, name: str, mode:
         # a caller that never collects: take the finished checks (no wait),
         # so the list stays bounded; an earlier bad id raises here
         raise_pending_id_errors(block=False)
-    bad = ((ids < 0) | (ids >= num_embeddings)).any().reshape(1)
+    if ids.dtype == torch.int64 and ids.numel() <= _ONE_BLOCK_IDS and num_embeddings > 0:
+        bad = _hip.ids_out_of_range(ids.contiguous(), num_embeddings)
+    else:
+        bad = ((ids < 0) | (ids >= num_embeddings)).any().reshape(1)
     host = torch.empty(1, dtype=torch.bool, pin_memory=True)
     host.copy_(bad, non_blocking=True)
     done = torch.cuda.Event()
