@@ -91,11 +91,32 @@ static GemmParams gate_params(const bf16_t* dY, const bf16_t* X, const CandGroup
     return p;
 }
 
+// Backward of up to kShortTokens tokens: the gate product's reduction runs over
+// the tokens, so its tiles are mostly epilogue, decodes of 65536 weights per
+// candidate, and two waves per SIMD hide each other's LDS reads and copies
+// where the four-wave tiles' one cannot.  Eight waves of 64x128 on 32x32x16
+// MFMAs, gate and dX in one launch.  Measured on MI355X, K = 6, backward
+// launches together, these against the four-wave stream: 6144 x 5120 at 61 /
+// 128 tokens 95 against 127, 98 against 119 us; 17408 x 5120 at 96-128 277
+// against 328, 1024 x 1024 31 against 38.  At 768 tokens they take 162 at 6144 x
+// 5120, and the stream 192 at 1024 where eight waves took 191; from 1536 on the
+// stream wins (631 against 640 at 17408 x 5120).
+constexpr int kShortTokens = 768;
+using ShortDxCfg = GemmCfg<DmaKS<256, 64, 512>, DmaNS<256, 64, 512>, 256, 256, 64, 4, 2, 2>;
+using ShortGateCfg =  // weight rows permuted for the gate epilogue
+    GemmCfg<DmaNS<256, 64, 512, 1>, DmaNS<256, 64, 512>, 256, 256, 64, 4, 2, 2, EPI_GATE>;
+
+static GemmParams short_dx_params(const bf16_t* dY, const bf16_t* W, int64_t ldw, bf16_t* dX, int M, int N, int D) {
+    GemmParams p{};
+    p.A = dY; p.lda = N; p.B = W; p.ldb = ldw; p.I = M; p.J = D; p.K = N; p.C = dX; p.ldc = D;
+    return p;
+}
+
 // One partial per gate grid block (split tail parts and idle padding blocks
 // included; the latter write zeros).
 int64_t gate_partial_count(int M, int N, int D) {
     GemmParams p = gate_params(nullptr, nullptr, CandGroup{}, nullptr, M, N, D);
-    return GateCfg::plan(p, device_cus(), true);
+    return M <= kShortTokens ? ShortGateCfg::plan(p, device_cus(), true) : GateCfg::plan(p, device_cus(), true);
 }
 
 // Gate products whose 256x256 dW tiles are few enough that the fused plan
@@ -142,7 +163,13 @@ int64_t gate_parts_bytes(int M, int N, int D) {
 int64_t dx_tail_bytes(int M, int N, int D) {
     GemmParams p = dx_params(nullptr, nullptr, 0, nullptr, M, N, D);
     DxCfg::plan(p, device_cus(), true);
-    return DxCfg::tail_bytes(p);
+    int64_t bytes = DxCfg::tail_bytes(p);
+    if (M <= kShortTokens) {
+        GemmParams q = short_dx_params(nullptr, nullptr, 0, nullptr, M, N, D);
+        ShortDxCfg::plan(q, device_cus(), true);
+        bytes = bytes > ShortDxCfg::tail_bytes(q) ? bytes : ShortDxCfg::tail_bytes(q);
+    }
+    return bytes;
 }
 
 // fp32 workspace for the K parts of the forward's split tail tiles: the most any
@@ -187,6 +214,11 @@ hipError_t launch_gemm_gate(const bf16_t* dY, const bf16_t* X, const CandGroup& 
         if (e != hipSuccess) return e;
         return launch_gate_dot(cg, N, D, dwp, np, partials, ds);
     }
+    if (M <= kShortTokens) {
+        const GemmParams p = gate_params(dY, X, cg, partials, M, N, D);
+        return any_iq(cg) ? launch_gemm_cfg<ShortGateCfg, true>(p, device_cus(), nullptr, s)
+                          : launch_gemm_cfg<ShortGateCfg>(p, device_cus(), nullptr, s);
+    }
     if (any_iq(cg))
         return launch_st_gate<GateCfg, true>(gate_params(dY, X, cg, partials, M, N, D), device_cus(), s);
     return launch_st_gate<GateCfg, false>(gate_params(dY, X, cg, partials, M, N, D), device_cus(), s);
@@ -206,6 +238,12 @@ hipError_t launch_gemm_dx_gate(const bf16_t* dY, const bf16_t* W, int64_t ldw, b
         if (e == hipSuccess) e = stream_fence(s, ds);
         if (e != hipSuccess) return e;
         return launch_gate_dot(cg, N, D, dwp, np, partials, ds);
+    }
+    if (M <= kShortTokens) {
+        const GemmParams x = short_dx_params(dY, W, ldw, dX, M, N, D);
+        const GemmParams g = gate_params(dY, X, cg, partials, M, N, D);
+        return any_iq(cg) ? launch_gemm_dual<ShortDxCfg, ShortGateCfg, true>(x, g, device_cus(), tail_ws, s)
+                          : launch_gemm_dual<ShortDxCfg, ShortGateCfg, false>(x, g, device_cus(), tail_ws, s);
     }
     if (any_iq(cg))
         return launch_st_dual<DxCfg, GateCfg, true>(dx_params(dY, W, ldw, dX, M, N, D),

@@ -111,8 +111,15 @@ struct DmaKS {
 // multiples of 32); the XOR moves the 4 k-rows' 64-byte blocks onto distinct
 // quarters of 256 bytes (as a 64-byte pad per k-row would).  The read at
 // k + 4 keeps the same XOR.
-template <int ROWS, int BK, int THREADS>
+// PERM = 1 reorders each 32-row fragment by 4-row granules: MFMA row 4 q + t
+// reads tile row 4 rot(q) + t, rot(q) = 4 (q % 2) + q / 2.  Accumulator
+// element 4 u + t of lane l (MFMA row 8 u + 4 (l / 32) + t) then holds tile
+// row 16 (l / 32) + 4 u + t: each lane's 16 values of a 32x32 block are 16
+// consecutive tile rows.  Each 32-lane half still reads whole 64-byte blocks
+// of the same 4 k-rows, so the reads stay conflict-free.
+template <int ROWS, int BK, int THREADS, int PERM = 0>
 struct DmaNS {
+    static constexpr int kPerm = PERM;
     static constexpr int kFragReads = 2;
     static constexpr int RCH = ROWS / 8;  // chunks per k-row
     static_assert(RCH % 16 == 0, "the XOR of up to 12 stays inside the k-row");
@@ -154,7 +161,7 @@ struct DmaNS {
         typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
         const int k = 16 * ks + 8 * (lane >> 5) + ((lane & 15) >> 2);
         const int q = 4 * ((lane >> 4) & 1) + (lane & 3);  // 4-row granule of the MFMA rows
-        const int r = row + 4 * q;
+        const int r = row + 4 * (PERM ? (((q & 1) << 2) | (q >> 1)) : q);
         const bf16_t* base =
             reinterpret_cast<const bf16_t*>(lds) + 8 * (k * RCH + ((r >> 3) ^ (4 * (k & 3)))) + (r & 7);
         const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(base));
@@ -397,12 +404,14 @@ __device__ __forceinline__ void gemm_mainloop_pp(const GemmParams& p, int i0, in
             if (ks == 0 && kt >= 1) issue_b(kt + 1);  // the B half of the refill issued at the last switch
         }
         __builtin_amdgcn_sched_group_barrier(0x100, FR, 0);  // reads of k-step 1 first
+        if constexpr (WI * WJ <= 4) {  // eight waves leave the rest of a stage to the scheduler
 #pragma unroll
-        for (int ks = 1; ks + 1 < KS; ++ks) {
+            for (int ks = 1; ks + 1 < KS; ++ks) {
 #pragma unroll
-            for (int r = 0; r < FR; ++r) {
-                __builtin_amdgcn_sched_group_barrier(0x008, (MF + FR - 1) / FR, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                for (int r = 0; r < FR; ++r) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, (MF + FR - 1) / FR, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                }
             }
         }
         __builtin_amdgcn_sched_group_barrier(0x008, MF, 0);
@@ -445,6 +454,177 @@ constexpr int kGateMaxChunks = gate_span_chunks(272);  // worst type (Q8_0)
 
 __device__ __forceinline__ int gate_row_chunks(int qt) { return gate_span_chunks(group_bytes(qt)); }
 
+// The eight-wave tiles' epilogue (short reductions; the four-wave one is in
+// vq_gemm_stream.h).
+template <int BJ, int THREADS>
+__device__ __forceinline__ void gate_stage_lds(u32x4* __restrict__ buf, const uint8_t* __restrict__ qbytes, int qt,
+                                               int64_t row_groups, int j0, int group, int J) {
+    typedef __attribute__((address_space(3))) void lds_void;
+    const int gb = group_bytes(qt), nch = gate_row_chunks(qt);
+    const int64_t origin = ((int64_t)j0 * row_groups * gb) & ~int64_t(15);
+    const int64_t bytes = (int64_t)J * row_groups * gb - origin;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(qbytes + origin), (short)0, (int)(bytes < (int64_t)kRange ? bytes : (int64_t)kRange),
+        0x00020000);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NW = THREADS / 64;
+    const int total = BJ * nch;
+    for (int base = wave * 64; base < total; base += NW * 64) {
+        const int id = base + lane;
+        const int row = id / nch, c = id % nch;
+        const int n = (j0 + row < J && id < total) ? j0 + row : j0;
+        const int64_t span = ((int64_t)n * row_groups + group) * gb;
+        // one instruction per wave: lanes land at buf + 16 (base + lane)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(buf + base), 16,
+                                                 (uint32_t)((span & ~int64_t(15)) - origin + 16 * c), 0, 0, 0);
+    }
+}
+
+// <acc, W_k> over the lane's accumulators: with the A operand's rows
+// permuted (DmaNS PERM = 1), block (a, b) holds, for row n = 32 b + lane%32,
+// the 16 consecutive weights 32 a + 16 (lane/32) + r, r = 0..15 (relative to
+// the wave's tile origin).
+template <int QT, int MI, int NJ, int WTI, int WTJ>
+__device__ __forceinline__ float gate_dot_lds(const f32x16 (&acc)[MI][NJ], const float (&sv)[MI][NJ],
+                                              const uint8_t* __restrict__ buf, int64_t row_groups, int j0, int group,
+                                              int wi, int wj, int lane, int J) {
+    constexpr int GB = group_bytes(QT);
+    constexpr int PITCH = 16 * gate_span_chunks(GB);  // bytes per staged row span
+    float s = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NJ; ++b) {
+        const int nl = wj * WTJ + 32 * b + (lane & 31);
+        // rows past J were staged from the tile's first row: locate their bytes the same way
+        const int n = j0 + nl < J ? j0 + nl : j0;
+        const int64_t span = ((int64_t)n * row_groups + group) * GB;
+        const uint8_t* g = buf + nl * PITCH + (int)(span & 15);
+#pragma unroll
+        for (int a = 0; a < MI; ++a) {
+            float v[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = acc[a][b][r];
+            s += dot_sub16<QT>(g, wi * WTI + 32 * a + 16 * (lane >> 5), v, sv[a][b]);
+            asm volatile("" : "+v"(lane), "+v"(s));  // one block's decode at a time
+        }
+    }
+    return s;
+}
+
+// gate_dot_lds for the IQ formats (type known at run time, uniform)
+template <int MI, int NJ, int WTI, int WTJ>
+__device__ __forceinline__ float gate_dot_lds_iq(int qt, const f32x16 (&acc)[MI][NJ], const float (&sv)[MI][NJ],
+                                                 const uint8_t* __restrict__ buf, int64_t row_groups, int j0,
+                                                 int group, int wi, int wj, int lane, int J) {
+    const int gb = group_bytes(qt);
+    const int pitch = 16 * gate_span_chunks(gb);
+    float s = 0.0f;
+#pragma unroll
+    for (int b = 0; b < NJ; ++b) {
+        const int nl = wj * WTJ + 32 * b + (lane & 31);
+        const int n = j0 + nl < J ? j0 + nl : j0;
+        const int64_t span = ((int64_t)n * row_groups + group) * gb;
+        const uint8_t* g = buf + nl * pitch + (int)(span & 15);
+#pragma unroll
+        for (int a = 0; a < MI; ++a) {
+            float v[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = acc[a][b][r];
+            s += dot_sub16_iq(qt, g, wi * WTI + 32 * a + 16 * (lane >> 5), v, sv[a][b]);
+            asm volatile("" : "+v"(lane), "+v"(s));  // one block's decode at a time
+        }
+    }
+    return s;
+}
+
+// IQ: the candidate set may hold IQ formats (their table-lookup decode needs
+// registers the K-quant-only instantiation keeps for itself).
+template <int BI, int BJ, int BK, int WI, int WJ, bool IQ>
+__device__ __forceinline__ void gate_epilogue(const GemmParams& p, int block, int i0, int j0,
+                                              u32x4* __restrict__ smem,
+                                              const f32x16 (&acc)[GemmShape<BI, BJ, BK, WI, WJ>::MI]
+                                                                 [GemmShape<BI, BJ, BK, WI, WJ>::NJ]) {
+    using S = GemmShape<BI, BJ, BK, WI, WJ>;
+    static_assert(BI == 256, "the gate tile covers exactly one 256-weight group per row");
+    constexpr int NW = WI * WJ;
+    constexpr int BUF_CH = BJ * kGateMaxChunks;  // 16-byte chunks per candidate buffer
+    // per-wave candidate sums, after the two candidate buffers (inside the
+    // dynamic allocation: a static array would push an 8-wave workgroup whose
+    // main loop takes all 160 KiB past the limit)
+    float(*red)[kMaxCand] = reinterpret_cast<float(*)[kMaxCand]>(smem + 2 * BUF_CH);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scale fields index by it
+    const int wi = wave / WJ, wj = wave % WJ;
+    const int group = i0 / 256;
+    // the gated tensor this tile's rows belong to (uniform per block)
+    int g = 0;
+#pragma unroll
+    for (int q = 1; q < kMaxSets; ++q)
+        if (q < p.cg.nsets && j0 >= p.cg.set_j0[q]) g = q;
+    const CandSet& cs = p.cg.sets[g];
+    const int jl0 = j0 - p.cg.set_j0[g];                 // first row within the tensor
+    const int jn = p.cg.set_j0[g + 1] - p.cg.set_j0[g];  // the tensor's rows
+    const int64_t rg = cs.row_groups;
+    // candidate-independent sums of each accumulator block
+    float sv[S::MI][S::NJ];
+#pragma unroll
+    for (int a = 0; a < S::MI; ++a)
+#pragma unroll
+        for (int b = 0; b < S::NJ; ++b) {
+            float t = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) t += acc[a][b][r];
+            sv[a][b] = t;
+        }
+    __syncthreads();  // every wave is past its last main-loop LDS read
+    gate_stage_lds<BJ, S::THREADS>(smem, cs.qbytes[0], cs.qtype[0], rg, jl0, group, jn);
+    for (int k = 0; k < cs.ncand; ++k) {
+        // this wave's direct-to-LDS copies of candidate k have landed, then
+        // everyone's have; buffer (k+1) % 2 is no longer read
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (k + 1 < cs.ncand)
+            gate_stage_lds<BJ, S::THREADS>(smem + ((k + 1) & 1) * BUF_CH, cs.qbytes[k + 1], cs.qtype[k + 1], rg, jl0,
+                                           group, jn);
+        const uint8_t* buf = reinterpret_cast<const uint8_t*>(smem + (k & 1) * BUF_CH);
+        // opaque per candidate: the decoders' field offsets and shifts are the
+        // same for each and would all be kept across the loop, spilling beside
+        // the accumulators
+        int ln = lane, wik = wi, wjk = wj;
+        asm volatile("" : "+v"(ln), "+s"(wik), "+s"(wjk));
+        float sum;
+        switch (cs.qtype[k]) {
+        case Q8_0: sum = gate_dot_lds<Q8_0, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wik, wjk, ln, jn); break;
+        case Q2_K: sum = gate_dot_lds<Q2_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wik, wjk, ln, jn); break;
+        case Q3_K: sum = gate_dot_lds<Q3_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wik, wjk, ln, jn); break;
+        case Q4_K: sum = gate_dot_lds<Q4_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wik, wjk, ln, jn); break;
+        case Q5_K: sum = gate_dot_lds<Q5_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wik, wjk, ln, jn); break;
+        default:
+            if constexpr (IQ) {
+                if (is_iq(cs.qtype[k])) {
+                    sum = gate_dot_lds_iq<S::MI, S::NJ, S::WTI, S::WTJ>(cs.qtype[k], acc, sv, buf, rg, jl0, group, wik,
+                                                                        wjk, ln, jn);
+                    break;
+                }
+            }
+            sum = gate_dot_lds<Q6_K, S::MI, S::NJ, S::WTI, S::WTJ>(acc, sv, buf, rg, jl0, group, wik, wjk, ln, jn);
+            break;
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
+        if (lane == 0) red[wave][k] = sum;
+    }
+    __syncthreads();
+    // this block's slots of every tensor: its own sums, zeros for the others
+    const int nslot = p.cg.nsets * p.cg.kstride;
+    if ((int)threadIdx.x < nslot) {
+        const int k = (int)threadIdx.x - g * p.cg.kstride;
+        float s = 0.0f;
+        if (k >= 0 && k < cs.ncand)
+            for (int wv = 0; wv < NW; ++wv) s += red[wv][k];
+        p.partials[(int64_t)block * nslot + threadIdx.x] = s;
+    }
+}
+
 // ---------------------------------------------------------------- kernels
 // K steps a split part of a store tile must save (see GemmCfg::plan).  14
 // against 10: the dual backward at 8192 tokens, 1024 -> 1536 (24 K steps of
@@ -452,9 +632,11 @@ __device__ __forceinline__ int gate_row_chunks(int qt) { return gate_span_chunks
 // 4096 -> 28672 and the other 1024-wide products.
 constexpr int kMinSavedSplitSteps = 14;
 
-// One small-tile configuration: loaders, tile, wave layout.
-template <class LA_, class LB_, int BI_, int BJ_, int BK_, int WI_, int WJ_, int OCC_>
+// One configuration: loaders, tile, wave layout, occupancy, epilogue.
+template <class LA_, class LB_, int BI_, int BJ_, int BK_, int WI_, int WJ_, int OCC_, int EPI_ = EPI_STORE>
 struct GemmCfg {
+    static_assert(EPI_ == EPI_STORE || EPI_ == EPI_GATE, "no parts");
+    static constexpr int EPI = EPI_;
     using LA = LA_;
     using LB = LB_;
     static constexpr int BI = BI_, BJ = BJ_, BK = BK_, WI = WI_, WJ = WJ_;
@@ -462,8 +644,11 @@ struct GemmCfg {
     static constexpr int THREADS = WI * WJ * 64;
     static constexpr size_t lds() {
         constexpr size_t store = (size_t)BI * (BJ + 8) * 2;  // bf16 staging of the tile
+        // two candidate buffers, wave sums
+        constexpr size_t gate = (size_t)2 * BJ * kGateMaxChunks * 16 + (size_t)WI * WJ * kMaxCand * 4;
+        constexpr size_t epi = EPI == EPI_GATE ? gate : store;
         constexpr size_t main = StageLds<LA, LB, 2>::BYTES;
-        return store > main ? store : main;
+        return epi > main ? epi : main;
     }
     static int tiles_i(const GemmParams& p) { return (p.I + BI - 1) / BI; }
     static int tiles_j(const GemmParams& p) { return (p.J + BJ - 1) / BJ; }
@@ -473,7 +658,7 @@ struct GemmCfg {
         if (p.I <= 0 || p.J <= 0) return 0;
         // a split store tile pays for its partial writes and a fixup launch:
         // split only when a part saves at least kMinSavedSplitSteps K steps
-        p.split_min_saved = kMinSavedSplitSteps;
+        p.split_min_saved = EPI == EPI_STORE ? kMinSavedSplitSteps : 0;
         p.split_max = 8;
         p.cus_per_xcd = cus / 8 > 0 ? cus / 8 : 1;
         p.split_ok = split_ok ? 1 : 0;
@@ -542,8 +727,9 @@ __device__ __forceinline__ void store_tile_lds(const GemmParams& p, int i0, int 
     }
 }
 
-// Work item `block` of problem p.
-template <class C>
+// Work item `block` of problem p.  IQ: a gate product whose candidate sets
+// may hold IQ formats.
+template <class C, bool IQ = false>
 __device__ __forceinline__ void gemm_body(const GemmParams& p, int block, u32x4* __restrict__ smem) {
     using LA = typename C::LA;
     using LB = typename C::LB;
@@ -553,7 +739,13 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p, int block, u32x4*
     const int ksteps = (p.K + BK - 1) / BK;
     const WorkItem w = map_work(block, tiles_i, tiles_j, ksteps, p.cus_per_xcd, p.split_ok != 0, p.tail_max, kGroupM,
                                 p.split_min_saved, p.split_max);
-    if (w.idle) return;
+    if (w.idle) {
+        if constexpr (C::EPI == EPI_GATE) {
+            const int nslot = p.cg.nsets * p.cg.kstride;
+            if ((int)threadIdx.x < nslot) p.partials[(int64_t)block * nslot + threadIdx.x] = 0.0f;
+        }
+        return;
+    }
     const int i0 = w.tm * BI, j0 = w.tn * BJ;
     int kbeg = 0, kend = p.K;
     if (w.ns > 1) {
@@ -563,6 +755,11 @@ __device__ __forceinline__ void gemm_body(const GemmParams& p, int block, u32x4*
     }
     f32x16 acc[S::MI][S::NJ];
     gemm_mainloop_pp<LA, LB, BI, BJ, BK, WI, WJ>(p, i0, j0, kbeg, kend, smem, acc);
+    if constexpr (C::EPI == EPI_GATE) {
+        static_assert(LA::kPerm == 1, "the gate epilogue reads 16 consecutive weights per accumulator block");
+        gate_epilogue<BI, BJ, BK, WI, WJ, IQ>(p, block, i0, j0, smem, acc);
+        return;
+    }
     if (w.ns > 1) {
         // K part of a split tail tile: fp32 partial, [element][thread]
         float* slot = p.partials + ((int64_t)w.tail_slot * p.s_max + w.split) * (BI * BJ);
@@ -622,12 +819,30 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tail_fixup_kernel(GemmParams 
 // (OCC: two, for two 128x128 workgroups per CU): telling the compiler
 // so lets it keep fragments in flight instead of minimising registers for an
 // occupancy the LDS use rules out anyway.
-template <class C>
+template <class C, bool IQ = false>
 __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(C::OCC, C::OCC)))
 void gemm_kernel(GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass needs only the launch stub
     extern __shared__ u32x4 smem[];
-    gemm_body<C>(p, blockIdx.x, smem);
+    gemm_body<C, IQ>(p, blockIdx.x, smem);
+#endif
+}
+
+// Two independent products in one launch: blocks [0, n1) run problem 1, blocks
+// [n1, ...) problem 2 (n1 is a multiple of 8, so both keep the XCD mapping of
+// map_work).  One grid lets the second product's work items fill the last,
+// partial round of the first.
+template <class C1, class C2, bool IQ1>
+__global__ __launch_bounds__(C1::THREADS) __attribute__((amdgpu_waves_per_eu(C1::OCC, C1::OCC)))
+void gemm_dual_kernel(GemmParams p1, int n1, GemmParams p2) {
+    static_assert(C1::THREADS == C2::THREADS && C1::OCC == C2::OCC, "both problems use the same workgroup shape");
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass needs only the launch stub
+    extern __shared__ u32x4 smem[];
+    const int b = blockIdx.x;
+    if (b < n1)
+        gemm_body<C1, IQ1>(p1, b, smem);
+    else
+        gemm_body<C2>(p2, b - n1, smem);
 #endif
 }
 
@@ -642,24 +857,48 @@ static hipError_t set_lds_attr(const void* kern, size_t lds, bool& done) {
     return e;
 }
 
-// Launch of one product.  `cus` is the device's CU count; tail tiles are split
-// only when `tail_ws` (tail_bytes of the plan) is given.
-template <class C>
+// Launch of one product.  `cus` is the device's CU count; a store epilogue
+// splits tail tiles only when `tail_ws` (tail_bytes of the plan) is given.
+template <class C, bool IQ = false>
 static hipError_t launch_gemm_cfg(GemmParams p, int cus, float* tail_ws, hipStream_t s) {
-    const int grid = C::plan(p, cus, tail_ws != nullptr);
+    const int grid = C::plan(p, cus, C::EPI == EPI_GATE || tail_ws != nullptr);
     if (grid == 0) return hipSuccess;
-    p.partials = tail_ws;
+    if (C::EPI == EPI_STORE) p.partials = tail_ws;
     constexpr size_t lds = C::lds();
     static_assert(lds <= 160 * 1024, "exceeds the 160 KiB of LDS per workgroup");
     static bool attr_set = false;  // per instantiation
-    auto kern = gemm_kernel<C>;
+    auto kern = gemm_kernel<C, IQ>;
     hipError_t e = set_lds_attr<C>((const void*)kern, lds, attr_set);
     if (e != hipSuccess) return e;
     kern<<<dim3(grid), dim3(C::THREADS), lds, s>>>(p);
     e = hipGetLastError();
-    if (e != hipSuccess || p.tail_max == 0) return e;
+    if (e != hipSuccess || C::EPI != EPI_STORE || p.tail_max == 0) return e;
     constexpr int FIX_BLOCKS = GemmShape<C::BI, C::BJ, C::BK, C::WI, C::WJ>::MI * GemmShape<C::BI, C::BJ, C::BK, C::WI, C::WJ>::NJ;
     gemm_tail_fixup_kernel<C><<<dim3(8 * p.tail_max * FIX_BLOCKS), dim3(C::THREADS), 0, s>>>(p);
+    return hipGetLastError();
+}
+
+// A gate product C2 and a store product C1 with split tails (tail_ws1, fixed
+// up after the launch) in one launch, the gate's work items first.
+template <class C1, class C2, bool IQ2>
+static hipError_t launch_gemm_dual(GemmParams p1, GemmParams p2, int cus, float* tail_ws1, hipStream_t s) {
+    static_assert(C1::EPI == EPI_STORE && C2::EPI == EPI_GATE, "a store product and a gate product");
+    const int grid1 = C1::plan(p1, cus, tail_ws1 != nullptr);
+    const int grid2 = C2::plan(p2, cus, true);
+    p1.partials = tail_ws1;
+    if (grid1 == 0) return launch_gemm_cfg<C2, IQ2>(p2, cus, nullptr, s);
+    if (grid2 == 0) return launch_gemm_cfg<C1>(p1, cus, tail_ws1, s);
+    constexpr size_t lds = C1::lds() > C2::lds() ? C1::lds() : C2::lds();
+    static_assert(lds <= 160 * 1024, "exceeds the 160 KiB of LDS per workgroup");
+    static bool attr_set = false;
+    auto kern = gemm_dual_kernel<C2, C1, IQ2>;
+    hipError_t e = set_lds_attr<C2>((const void*)kern, lds, attr_set);
+    if (e != hipSuccess) return e;
+    kern<<<dim3(grid2 + grid1), dim3(C2::THREADS), lds, s>>>(p2, grid2, p1);
+    e = hipGetLastError();
+    if (e != hipSuccess || p1.tail_max == 0) return e;
+    using S1 = GemmShape<C1::BI, C1::BJ, C1::BK, C1::WI, C1::WJ>;
+    gemm_tail_fixup_kernel<C1><<<dim3(8 * p1.tail_max * S1::MI * S1::NJ), dim3(C1::THREADS), 0, s>>>(p1);
     return hipGetLastError();
 }
 
