@@ -183,8 +183,9 @@ int check_bwd(const uint16_t* dy, const uint16_t* x, int64_t m, int64_t n, int64
 // allow_parts: the fused epilogue and its partials only.
 struct GateWs {
     bool parts;
+    bool few;            // a few tokens' own gate product (no parts; needs dwp_bytes too)
     int64_t part_bytes;  // 256-aligned partial area
-    int64_t dwp_bytes;   // 256-aligned parts area (0 without allow_parts or parts)
+    int64_t dwp_bytes;   // 256-aligned parts area, or few's copies (0 without allow_parts)
 };
 
 GateWs gate_ws(int64_t m, int64_t d, int64_t d_pad, int nsets, const int64_t* n, int64_t n_total, int nslot,
@@ -194,8 +195,13 @@ GateWs gate_ws(int64_t m, int64_t d, int64_t d_pad, int nsets, const int64_t* n,
     const bool possible = allow_parts && vq::gate_parts((int)m, (int)n_total, (int)d) > 0;
     const int64_t dot = possible ? vq::gate_dot_blocks(nsets, n, (d + 255) / 256) : 0;
     g.parts = possible && d_pad == (d + 255) / 256 * 256;
-    g.part_bytes = align256((fused > dot ? fused : dot) * nslot * (int64_t)sizeof(float));
-    g.dwp_bytes = possible ? align256(vq::gate_parts_bytes((int)m, (int)n_total, (int)d)) : 0;
+    g.few = allow_parts && nsets == 1 && !possible && vq::gate_few(m, n_total, d);
+    const int64_t few = g.few ? vq::gate_few_blocks(n_total, d) : 0;
+    const int64_t most = fused > dot ? fused : dot;
+    g.part_bytes = align256((most > few ? most : few) * nslot * (int64_t)sizeof(float));
+    g.dwp_bytes = possible ? align256(vq::gate_parts_bytes((int)m, (int)n_total, (int)d))
+                : g.few    ? align256(vq::gate_few_bytes(m, n_total, d))
+                           : 0;
     return g;
 }
 
@@ -213,6 +219,7 @@ int run_bwd(const uint16_t* dy, const uint16_t* x, int64_t m, int64_t n, int64_t
     const int ncand = cs.ncand;
     // the parts path when the shape takes it and its buffer is there
     float* parts = gw.parts ? dwp : nullptr;
+    const bool few = gw.few && dwp && dprobs && !dx && m > 0;
     if (dx) {
         const uint16_t* w = w_eff;
         if (remix_buf) {
@@ -239,14 +246,19 @@ int run_bwd(const uint16_t* dy, const uint16_t* x, int64_t m, int64_t n, int64_t
             if (rc == VQ_OK) rc = hip_check(vq::launch_gate_reduce(partials, 0, ncand, dprobs, gs), "gate reduce launch");
             return rc == VQ_OK ? ok() : rc;
         }
-        if (!dx) {
+        if (few) {
+            rc = hip_check(vq::launch_gate_few(dy, x, cs, partials, (int)m, (int)n, (int)d, dwp, s),
+                           "few-token gate launch");
+            if (rc != VQ_OK) return rc;
+        } else if (!dx) {
             rc = hip_check(
                 vq::launch_gemm_gate(dy, x, group_of(cs, n), partials, (int)m, (int)n, (int)d, parts, s, gs),
                 "gate GEMM launch");
             if (rc != VQ_OK) return rc;
         }
         // partials: one per dot block on the parts path, one per gate block otherwise
-        const int64_t nparts = parts ? vq::gate_dot_blocks(1, &n, d_pad / 256)
+        const int64_t nparts = few     ? vq::gate_few_blocks(n, d)
+                             : parts ? vq::gate_dot_blocks(1, &n, d_pad / 256)
                                      : vq::gate_partial_count((int)m, (int)n, (int)d);
         rc = hip_check(vq::stream_fence(s, gs), "stream fence");
         if (rc != VQ_OK) return rc;
@@ -775,7 +787,7 @@ int vq_gated_linear_bwd_gate_stream(const uint16_t* dy, const uint16_t* x, int64
     float* tail_ws = nullptr;
     if (workspace && tail_bytes > 0 && ws_bytes >= part_bytes + tail_bytes)
         tail_ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + part_bytes);
-    float* dwp = gw.parts && workspace && ws_bytes >= need
+    float* dwp = (gw.parts || gw.few) && workspace && ws_bytes >= need
                      ? reinterpret_cast<float*>(static_cast<char*>(workspace) + part_bytes + tail_bytes)
                      : nullptr;
     uint16_t* remix_buf = nullptr;
@@ -950,7 +962,7 @@ int vq_gated_linear_group_bwd_gate_stream(const uint16_t* dy, const uint16_t* x,
     float* tail_ws = nullptr;
     if (workspace && tail_bytes > 0 && ws_bytes >= part_bytes + tail_bytes)
         tail_ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + part_bytes);
-    float* dwp = gw.parts && workspace && ws_bytes >= need
+    float* dwp = (gw.parts || gw.few) && workspace && ws_bytes >= need
                      ? reinterpret_cast<float*>(static_cast<char*>(workspace) + part_bytes + tail_bytes)
                      : nullptr;
     // every member in one reduce; no tokens: a reduce over zero partials

@@ -84,6 +84,15 @@ hipError_t launch_gemm_dx_gate(const bf16_t* dY, const bf16_t* W, int64_t ldw, b
 // dW[n][d] * W_k[n][d], dW the sum of the parts dwp in part order
 hipError_t launch_gate_dot(const CandGroup& cg, int N, int D, const float* dwp, int parts, float* partials,
                            hipStream_t s);
+// Gate product of at most kFewGateTokens tokens (vq_gate_few.hip): partials
+// of gate_few_blocks blocks, ws: gate_few_bytes for the token-contiguous copies
+// of X and dY.
+constexpr int kFewGateTokens = 64;
+bool gate_few(int64_t M, int64_t N, int64_t D);
+int64_t gate_few_blocks(int64_t N, int64_t D);
+int64_t gate_few_bytes(int64_t M, int64_t N, int64_t D);
+hipError_t launch_gate_few(const bf16_t* dY, const bf16_t* X, const CandSet& cs, float* partials, int M, int N, int D,
+                           void* ws, hipStream_t s);
 // PTQR: Y[perm[r]] = X[perm[r]] . W_g^T for r in [group_off[g], group_off[g+1])
 hipError_t launch_routed_fwd(const bf16_t* X, int M, int D, const bf16_t* const* cand_bf16, int64_t ldw, int N,
                              int ncand, const int* perm, const int* group_off, bf16_t* Y, hipStream_t s);
