@@ -86,3 +86,28 @@ def test_gate_gradient_ignores_padding():
         _hip.gated_linear_bwd(dy, x, [8], [qq.reshape(-1).cuda()], None, n, d_pad, None, None, dp, ws)
         out.append(dp.cpu())
     assert torch.equal(out[0], out[1]) and torch.isfinite(out[0]).all()
+
+
+def test_group_of_one_member():
+    """A stack of one member takes the tiles, whatever the token count, and gives the same gradient."""
+    from voodoo_quant import _hip
+
+    m, n, d = 7, 256, 512
+    g = torch.Generator().manual_seed(9)
+    q = torch.randint(0, 256, (n * d // 32, 34), dtype=torch.uint8, generator=g)
+    q[:, 1] = 0x28
+    qd = q.reshape(-1).cuda()
+    x, dy = (torch.randn(m, c, generator=g).to(torch.bfloat16).cuda() for c in (d, n))
+    one = torch.empty(1, device="cuda")
+    ws = torch.empty(_hip.bwd_workspace_bytes(m, n, d, d, 1, False), dtype=torch.uint8, device="cuda")
+    _hip.gated_linear_bwd(dy, x, [8], [qd], None, n, d, None, None, one, ws)
+    members = [((8,), [qd], n)]
+    stacked = torch.empty(1, device="cuda")
+    ws = torch.empty(_hip.group_bwd_workspace_bytes(m, d, members), dtype=torch.uint8, device="cuda")
+    _hip.gated_linear_group_bwd(dy, x, members, d, None, None, [stacked], ws)
+    w = torch.from_numpy(cdequant.oracle_dequant("Q8_0", q.numpy(), n * d).reshape(n, d)).double()
+    dw = dy.double().cpu().t() @ x.double().cpu()
+    mags = dy.double().abs().cpu().t() @ x.double().abs().cpu()
+    scale = (mags * w.abs().max()).sum()
+    for got in (one, stacked):
+        assert (got.double().cpu() - (dw * w).sum()).abs() <= (m + 64) * 2.0**-24 * 4 * scale

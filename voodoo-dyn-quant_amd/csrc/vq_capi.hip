@@ -962,7 +962,7 @@ int vq_gated_linear_group_bwd_gate_stream(const uint16_t* dy, const uint16_t* x,
     float* tail_ws = nullptr;
     if (workspace && tail_bytes > 0 && ws_bytes >= part_bytes + tail_bytes)
         tail_ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + part_bytes);
-    float* dwp = (gw.parts || gw.few) && workspace && ws_bytes >= need
+    float* dwp = gw.parts && workspace && ws_bytes >= need
                      ? reinterpret_cast<float*>(static_cast<char*>(workspace) + part_bytes + tail_bytes)
                      : nullptr;
     // every member in one reduce; no tokens: a reduce over zero partials
